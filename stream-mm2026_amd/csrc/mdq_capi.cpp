@@ -504,6 +504,9 @@ int run_grad_stats(const void *const *grads, const int64_t *numels, int n, int g
     for (int i = 0; i < n; ++i) {
         if (numels[i] < 0) return fail(STQ_ERR_INVALID, "tensor %d: negative numel", i);
         if (numels[i] > 0 && !grads[i]) return fail(STQ_ERR_INVALID, "tensor %d: null grad", i);
+        // the kernel finds a tensor's place in its first line by element counts
+        if (numels[i] > 0 && !is_aligned(grads[i], grad_dt == STQ_FLOAT ? 4 : 2))
+            return fail(STQ_ERR_INVALID, "tensor %d: grad must be aligned to its element size", i);
         d[i].g = grads[i];
         d[i].numel = numels[i];
         d[i].tile_begin = tiles;

@@ -80,6 +80,35 @@ def test_thousands_of_small_tensors_one_launch():
         np.testing.assert_allclose(got[i], ref, rtol=1e-6, atol=0, equal_nan=True, err_msg=f"tensor {i} n={n}")
 
 
+@pytest.mark.parametrize("dtype,offsets", [(torch.float32, (0, 1, 3, 4, 17, 31)), (torch.bfloat16, (0, 1, 7, 8, 33, 63)),
+                                           (torch.float16, (1, 2, 62))])
+@pytest.mark.parametrize("values", ["spread", "mean", "tiny"])
+def test_tiles_at_any_place_in_their_line(dtype, offsets, values):
+    """Whole and ragged tiles that start at element 0 .. 31 (63) of a 128-byte line, NaN on both sides
+    of each view: values whose M2 comes from the plain sums, from the deviations (a mean that dwarfs
+    the spread) and from the fp64 redo (squares below fp32's normal range)."""
+    print(f"case: grad_stats places {dtype} {values}", flush=True)
+    rng = np.random.default_rng(7)
+    vs = []
+    for off in offsets:
+        for n in (32768, 32768 + 65536, 32767, 32768 - off, 32769, 5, 1000):
+            x = rng.standard_t(3, n) * 1e-3
+            if values == "mean":
+                x = 1.0 + x * 2.0 ** -4
+            elif values == "tiny":
+                x = rng.choice([-1.0, 1.0], n) * 2.0 ** (-75 if dtype != torch.float16 else -20)
+            buf = torch.full((n + 256,), float("nan"), dtype=dtype, device=DEV)
+            assert buf.data_ptr() % 128 == 0
+            buf[64 + off:64 + off + n] = torch.from_numpy(x).to(dtype).to(DEV)
+            vs.append(buf[64 + off:64 + off + n])
+    got = mdq_hip.grad_stats(vs).cpu().numpy()
+    again = mdq_hip.grad_stats(vs).cpu().numpy()
+    assert np.array_equal(got.view(np.uint32), again.view(np.uint32)), "not deterministic"
+    for i, v in enumerate(vs):
+        ref = orc.grad_stats(v.float().cpu().numpy())
+        np.testing.assert_allclose(got[i], ref, rtol=1e-6, atol=0, err_msg=f"view {i} n={v.numel()}")
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_nonfinite_grads_match_oracle(dtype):
     """NaN, +-inf and (fp32) overflowing squares in some tensors of a launch: the kernel gives the
