@@ -195,6 +195,28 @@ int stq_multi_tensor_mdq_adamw_noalloc(const stq_tensor *tensors, int n_tensors,
 int stq_multi_tensor_grad_stats(const void *const *grads, const int64_t *numels, int n_tensors,
                                 int grad_dtype, float *stats, void *stream);
 
+/*
+ * The scores of the MDQ bit decision from the statistics of n_tensors tensors
+ * (stats[3 n_tensors], as stq_multi_tensor_grad_stats writes them) and their
+ * mean over the tensors (mean[3], formed by the caller: across ranks it is
+ * reduced first), one launch:
+ *   ema[3] = alpha * mean + one_minus_alpha * (n_ema, r_ema, v_ema), or mean
+ *            where those three are NULL (the first decision);
+ *   out[i] = 7.2 + log2(r_l / (ema[1] + 1e-12)) + log2(n_l / (ema[0] + 1e-12))
+ *            + log2(1 + 1 / cosh(t[i])) + log2(v_l / (ema[2] + 1e-12)), every
+ *            operation rounded to fp32 in that order;
+ *   out[n_tensors + i] = r_l.
+ * t[i] = step / tau per tensor, or NULL where all tensors share t_all.  All
+ * arrays are device memory; out (2 n_tensors floats) and ema must not overlap
+ * the inputs.
+ *
+ * Replaces the per-tensor score of MDQAdamWSimple
+ * (/root/reference/CUDA/stquant_opt_simple.py:433-466).
+ */
+int stq_decision_scores(const float *stats, const float *mean, int n_tensors, const float *t, float t_all,
+                        const float *n_ema, const float *r_ema, const float *v_ema, float alpha,
+                        float one_minus_alpha, float *out, float *ema, void *stream);
+
 /* Code storage classes of stq_code_convert (the m/v code layouts the step kernels read). */
 enum {
     STQ_STORE_P4 = 0,   /* uint8 bytes (v << 4) | (m + 8), no separate v array */

@@ -921,6 +921,21 @@ int stq_multi_tensor_grad_stats(const void *const *grads, const int64_t *numels,
     return run_grad_stats(grads, numels, n_tensors, grad_dtype, stats, reinterpret_cast<hipStream_t>(stream));
 }
 
+int stq_decision_scores(const float *stats, const float *mean, int n_tensors, const float *t, float t_all,
+                        const float *n_ema, const float *r_ema, const float *v_ema, float alpha,
+                        float one_minus_alpha, float *out, float *ema, void *stream)
+{
+    g_err.clear();
+    if (n_tensors < 0 || (n_tensors > 0 && (!stats || !mean || !out || !ema)))
+        return fail(STQ_ERR_INVALID, "decision_scores: bad statistics or output");
+    if ((n_ema == nullptr) != (r_ema == nullptr) || (n_ema == nullptr) != (v_ema == nullptr))
+        return fail(STQ_ERR_INVALID, "decision_scores: all three EMAs or none");
+    if (n_tensors == 0) return STQ_OK;
+    const hipError_t e = mdq::launch_scores(stats, mean, n_tensors, t, t_all, n_ema, r_ema, v_ema, alpha,
+                                            one_minus_alpha, out, ema, reinterpret_cast<hipStream_t>(stream));
+    return e == hipSuccess ? STQ_OK : hip_fail(e, "decision_scores launch");
+}
+
 int stq_multi_tensor_convert_codes(const stq_code_convert *items, int n_tensors, void *stream)
 {
     return run_convert(items, n_tensors, reinterpret_cast<hipStream_t>(stream));

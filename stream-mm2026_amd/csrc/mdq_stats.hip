@@ -31,6 +31,8 @@
 //      large |mean| is against the spread.  The results are rounded to the
 //      reference's fp32 outputs.  A sum whose exact value exceeds FLT_MAX gives
 //      inf, as the reference's fp32 accumulators overflow.
+//   3. scores_kernel (a call of its own, after the caller's mean over the tensors):
+//      one thread per tensor folds the mean into the EMAs and forms the tensor's score.
 // Both orders are fixed by the tensor list, so results are deterministic.
 #include <hip/hip_runtime.h>
 
@@ -403,7 +405,49 @@ __global__ __launch_bounds__(ST_THREADS) void stats_finish_kernel(const StatDesc
     }
 }
 
+// The scores of the bit decision (stquant_opt_simple.py:433-466): the EMAs with this
+// decision's mean statistics folded in (the mean itself at the first decision), and per
+// tensor 7.2 + log2(r_l / (r + 1e-12)) + log2(n_l / (n + 1e-12)) + log2(1 + 1 / cosh t)
+// + log2(v_l / (v + 1e-12)), each operation rounded to fp32 in that order, so the bits are
+// those of the same chain of torch operations (checked in tests/test_gpu_grad_stats.py).
+// Bound by launches: as torch operations the chain is 24 of them, about 5 us of host time
+// each.  A width-deciding optimizer step over GPT-2 small's 148 tensors 1776 -> 1387 us with
+// this launch, once where the provisional scores settle no row, in place of the chain run twice.
+__global__ __launch_bounds__(256) void scores_kernel(const float *__restrict__ stats, const float *__restrict__ mean,
+                                                     int n, const float *__restrict__ t, float t_all,
+                                                     const float *__restrict__ n_ema, const float *__restrict__ r_ema,
+                                                     const float *__restrict__ v_ema, float a, float b,
+                                                     float *__restrict__ out, float *__restrict__ ema)
+{
+    const float en = n_ema ? a * mean[0] + b * *n_ema : mean[0];
+    const float er = n_ema ? a * mean[1] + b * *r_ema : mean[1];
+    const float ev = n_ema ? a * mean[2] + b * *v_ema : mean[2];
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i == 0) {
+        ema[0] = en;
+        ema[1] = er;
+        ema[2] = ev;
+    }
+    if (i >= n) return;
+    const float n_l = stats[3 * i], r_l = stats[3 * i + 1], v_l = stats[3 * i + 2];
+    const float s_t = 1.0f + 1.0f / coshf(t ? t[i] : t_all);
+    float s = 7.2f + log2f(r_l / (er + 1e-12f));
+    s = s + log2f(n_l / (en + 1e-12f));
+    s = s + log2f(s_t);
+    s = s + log2f(v_l / (ev + 1e-12f));
+    out[i] = s;
+    out[n + i] = r_l;
+}
+
 }  // namespace
+
+hipError_t launch_scores(const float *stats, const float *mean, int n, const float *t, float t_all, const float *n_ema,
+                         const float *r_ema, const float *v_ema, float a, float b, float *out, float *ema, hipStream_t s)
+{
+    scores_kernel<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s>>>(stats, mean, n, t, t_all, n_ema, r_ema, v_ema,
+                                                                         a, b, out, ema);
+    return hipGetLastError();
+}
 
 hipError_t launch_grad_stats(const StatDesc *d, const long long *tb, int n, long long tiles, int grad_dt,
                              double *partials, float *out, hipStream_t s)

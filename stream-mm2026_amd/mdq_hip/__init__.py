@@ -22,7 +22,7 @@ from .storage import layout_of as storage_of
 __all__ = [
     "ROUND_NEAREST", "ROUND_STOCHASTIC", "STORE_P4", "STORE_S8", "STORE_S16", "STORE_S32",
     "TensorState", "MultiTensorPlan", "fused_step", "multi_tensor_step", "multi_tensor_restore",
-    "RESTORE_BLOCK_SIZES", "grad_stats", "step_table_uploads", "convert_codes", "empty_codes", "storage_of",
+    "RESTORE_BLOCK_SIZES", "grad_stats", "decision_scores", "step_table_uploads", "convert_codes", "empty_codes", "storage_of",
     "block_aligned_ranges", "shard_states",
     "device_math", "device_math_digests", "device_log_approx_error", "device_hw_ulp_error", "host_math",
     "host_round_half_away",
@@ -424,6 +424,33 @@ def grad_stats(grads: Sequence[torch.Tensor], out: Optional[torch.Tensor] = None
             if dst is not out:
                 out[torch.as_tensor(idx, device=dev)] = dst
     return out
+
+
+def decision_scores(stats: torch.Tensor, mean: torch.Tensor, t: Sequence[float], ema, alpha: float):
+    """The bit decision's scores of the tensors with statistics ``stats`` (``[n, 3]``, as
+    ``grad_stats`` gives them), in one launch: ``(scores_and_r, ema)``, a ``[2 n]`` device tensor
+    of the n scores and the n ``r_l``, and the ``[3]`` EMAs (n, r, v) after folding in ``mean``.
+    ``t``: each tensor's step / tau; ``ema``: the EMAs so far (three 0-d tensors), or None at the
+    first decision.  The same fp32 operations as the reference's (stquant_opt_simple.py:433-466)."""
+    n, dev = stats.shape[0], stats.device
+    if dev.type != "cuda" or len(t) != n:
+        raise RuntimeError("decision_scores: statistics on a CUDA device and one t per tensor")
+    for x in (stats, mean) + tuple(ema or ()):
+        if x.dtype != torch.float32 or x.device != dev or not x.is_contiguous():
+            raise RuntimeError("decision_scores: statistics, mean and EMAs must be contiguous float32 on one device")
+    if mean.numel() != 3 or (ema is not None and any(x.numel() != 1 for x in ema)):
+        raise RuntimeError("decision_scores: a mean of 3 and three EMAs")
+    out = torch.empty(2 * n, dtype=torch.float32, device=dev)
+    new = torch.empty(3, dtype=torch.float32, device=dev)
+    if n == 0:
+        return out, new
+    same = t.count(t[0]) == n
+    ts = None if same else torch.tensor(t, dtype=torch.float32, device=dev)
+    e = [x.data_ptr() for x in ema] if ema is not None else [None] * 3
+    with torch.cuda.device(dev):
+        check(lib().stq_decision_scores(stats.data_ptr(), mean.data_ptr(), n, _ptr(ts), t[0], *e, alpha, 1 - alpha,
+                                        out.data_ptr(), new.data_ptr(), _capi.stream_handle(dev)))
+    return out, new
 
 
 # stq_code_convert: 4 pointers, int64 numel, two int32 storages (48 bytes)

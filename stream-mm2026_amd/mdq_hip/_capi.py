@@ -38,6 +38,7 @@ EXPORTED_SYMBOLS = (
     "stq_multi_tensor_mdq_adamw_noalloc",
     "stq_multi_tensor_mdq_adamw_restore",
     "stq_multi_tensor_grad_stats",
+    "stq_decision_scores",
     "stq_multi_tensor_convert_codes",
     "stq_last_error",
     "stq_abi_version",
@@ -125,6 +126,8 @@ def lib() -> ctypes.CDLL:
     L.stq_multi_tensor_convert_codes.restype = ctypes.c_int
     L.stq_multi_tensor_grad_stats.argtypes = [vp, vp, i32, i32, vp, vp]
     L.stq_multi_tensor_grad_stats.restype = ctypes.c_int
+    L.stq_decision_scores.argtypes = [vp, vp, i32, vp, f32, vp, vp, vp, f32, f32, vp, vp, vp]
+    L.stq_decision_scores.restype = ctypes.c_int
     L.stq_last_error.argtypes = []
     L.stq_last_error.restype = ctypes.c_char_p
     L.stq_abi_version.argtypes = []

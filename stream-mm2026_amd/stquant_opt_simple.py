@@ -194,32 +194,53 @@ class MDQAdamWSimple(Optimizer):
         """``[n, 3]`` stats of all grads: one fused launch per grad dtype (``'fused'``, settled on
         the reference's torch reductions near the thresholds, and ``'exact'``), or the reference's
         per-tensor torch reductions (``'reference'``, stquant_opt_simple.py:427-431)."""
+        return self._stats_and_decision(grads, steps, tau)[0]
+
+    def _stats_and_decision(self, grads, steps=None, tau=None):
+        """``_all_grad_stats``, and the decision (``_decision``) that settling them already made on
+        exactly these statistics (None where it made none, or on others)."""
         if self.grad_stats != "reference" and grads and grads[0].is_cuda:
             stats = mdq_hip.grad_stats(grads)
             if self.grad_stats == "fused" and steps is not None:
-                stats = self._settle(stats, grads, steps, tau)
-            return stats
-        return torch.stack([self._compute_grad_stats(g.float()) for g in grads])
+                return self._settle(stats, grads, steps, tau)
+            return stats, None
+        return torch.stack([self._compute_grad_stats(g.float()) for g in grads]), None
+
+    def _decision(self, stats, mean, steps, tau):
+        """``(scores, host, ema)`` of these statistics and their mean, which the EMAs fold in: the
+        ``[n]`` scores, a host array of them and the tensors' r_l, and the new EMAs (n, r, v).
+        One launch and one host read where the statistics are on a GPU; ``_folded_ema`` and
+        ``_scores``, the same operations in torch, otherwise."""
+        ema = None if self.n_ema is None else (self.n_ema, self.r_ema, self.v_global_ema)
+        n = stats.shape[0]
+        if stats.is_cuda and all(torch.is_tensor(x) and x.dtype == torch.float32 and x.device == stats.device
+                                 and x.numel() == 1 for x in ema or ()):
+            both, new = mdq_hip.decision_scores(stats, mean, [s / tau for s in steps], ema,
+                                                self.param_groups[0]["alpha"])
+            return both[:n], both.cpu().numpy(), new.unbind(0)
+        new = self._folded_ema(mean)
+        scores = self._scores(stats, steps, tau, ema=new)
+        return scores, torch.cat((scores, stats[:, 1])).cpu().numpy(), new
 
     def _settle(self, stats, grads, steps, tau):
         """The fused statistics, with the rows of the tensors whose width the fused and the
         reference statistics could decide differently replaced by the reference's torch
         reductions: scores within SETTLE_MARGIN of a threshold (provisional scores against the
-        EMAs this decision would fold in), near-constant tensors, and non-finite rows."""
-        prov = self._scores(stats, steps, tau, ema=self._folded_ema(stats.mean(dim=0)))
-        host = torch.cat((prov, stats[:, 1])).cpu().numpy()
-        sc, r = host[:len(grads)], host[len(grads):]
+        EMAs this decision would fold in), near-constant tensors, and non-finite rows.  With them
+        the provisional decision, where no row was replaced."""
+        prov = self._decision(stats, stats.mean(dim=0), steps, tau)
+        sc, r = prov[1][:len(grads)], prov[1][len(grads):]
         near = np.zeros(len(grads), dtype=bool)
         for _bits, lo in _WIDTH_THRESHOLDS:
             near |= np.abs(sc - lo) < self.SETTLE_MARGIN
         redo = np.nonzero(near | (r < self.NEAR_CONSTANT_R) | ~np.isfinite(sc) | ~np.isfinite(r))[0].tolist()
         if not redo:
-            return stats
+            return stats, prov
         stats = stats.clone()
         stats[torch.as_tensor(redo, device=stats.device)] = torch.stack(
             [self._compute_grad_stats(grads[i].float()) for i in redo])
         self._settled = len(redo)
-        return stats
+        return stats, None
 
     def _scores(self, stats_tensor, steps, tau, ema=None):
         """The reference's per-tensor score (stquant_opt_simple.py:446-466) for all tensors at
@@ -253,9 +274,6 @@ class MDQAdamWSimple(Optimizer):
         prev = torch.stack((self.n_ema, self.r_ema, self.v_global_ema))
         return (a * mean + (1 - a) * prev).unbind(0)
 
-    def _fold_ema(self, mean: torch.Tensor) -> None:
-        self.n_ema, self.r_ema, self.v_global_ema = self._folded_ema(mean)
-
     def _decide_bits(self, work) -> None:
         """Score every tensor with a grad against the global statistics and give the tensors of
         scored groups their width; fills the decision's timing keys."""
@@ -265,21 +283,22 @@ class MDQAdamWSimple(Optimizer):
         tau = self.param_groups[0]["tau"]
         self._settled = 0
         with _Stopwatch(dev) as sw:
-            stats = self._all_grad_stats([p.grad for p, _g in work], steps, tau)
+            stats, made = self._stats_and_decision([p.grad for p, _g in work], steps, tau)
         lt["mdq_grad_stats_ms"] = sw.ms
         lt["mdq_grad_stats_settled"] = self._settled
-        mean = stats.mean(dim=0)
-        if dist.is_available() and dist.is_initialized():
+        across = dist.is_available() and dist.is_initialized()
+        mean = stats.mean(dim=0) if across or made is None else None
+        if across:
             with _Stopwatch(dev) as sw:
                 dist.all_reduce(mean, op=dist.ReduceOp.SUM)
                 mean /= dist.get_world_size()
             lt["mdq_allreduce_ms"] = sw.ms
         with _Stopwatch(dev) as sw:
-            self._fold_ema(mean)
+            # settling's decision stands where it changed no row and no other rank has a say
+            scores, host, ema = made if mean is None else self._decision(stats, mean, steps, tau)
+            self.n_ema, self.r_ema, self.v_global_ema = ema
             states = [self.state[p] for p, _g in work]
-            scores = self._scores(stats, steps, tau)
-            host = scores.cpu().tolist()                 # the step's one device -> host read
-            for (_p, g), st, s, h in zip(work, states, scores.unbind(0), host):
+            for (_p, g), st, s, h in zip(work, states, scores.unbind(0), host.tolist()):
                 st["last_score"] = s
                 if g.get("bits") is None:
                     st["current_bit"] = self._score_to_bits(h)

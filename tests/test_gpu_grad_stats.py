@@ -166,6 +166,37 @@ def test_vectorised_score_is_the_reference_expression():
         assert opt._score_to_bits(float(vec[i].item())) == opt._score_to_bits(ref)
 
 
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 3001])
+@pytest.mark.parametrize("first,same_step", [(True, True), (False, True), (False, False)])
+def test_decision_launch_is_the_torch_chain(n, first, same_step):
+    """``decision_scores`` against ``_folded_ema`` and ``_scores``, bit for bit: statistics over the
+    whole fp32 range, zeros, inf and NaN among them, and step / tau from 0 to far past cosh's
+    overflow."""
+    print(f"case: decision_scores n={n} first={first} same_step={same_step}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(n)
+    opt = MDQAdamWSimple([torch.nn.Parameter(torch.zeros(8, device=DEV))], alpha=0.83)
+    stats = torch.randn(n, 3, device=DEV, generator=g).mul_(12).exp_()
+    special = torch.tensor([0.0, float("inf"), float("nan"), 1e-45, 3e38, 1e-38], device=DEV)
+    if n > 200:
+        stats[7:7 + len(special), 0] = special
+        stats[30:30 + len(special), 1] = special
+        stats[60:60 + len(special), 2] = special
+    mean = torch.rand(3, device=DEV, generator=g) * 1e-3
+    if not first:
+        opt.n_ema, opt.r_ema, opt.v_global_ema = (torch.rand(3, device=DEV, generator=g) * 1e-2).unbind(0)
+    steps = [1234] * n if same_step else [int(x) for x in np.random.default_rng(n).integers(1, 200_000, n)]
+    tau = 1717.3
+    scores, host, ema = opt._decision(stats, mean, steps, tau)
+    want_ema = opt._folded_ema(mean)
+    want = opt._scores(stats, steps, tau, ema=want_ema)
+    for got, ref in zip(ema, want_ema):
+        assert torch.equal(got.view(torch.int32), ref.view(torch.int32))
+    assert torch.equal(torch.isnan(scores), torch.isnan(want))
+    ok = ~torch.isnan(want)
+    assert torch.equal(scores[ok].view(torch.int32), want[ok].view(torch.int32))
+    np.testing.assert_array_equal(host, torch.cat((want, stats[:, 1])).cpu().numpy())
+
+
 def test_optimizer_fused_stats_same_decisions():
     print("case: optimizer grad_stats fused vs reference", flush=True)
     shapes = [(700, 13), (4096,), (129,), (3, 1000), (50_000,)]
