@@ -1249,22 +1249,17 @@ __device__ __forceinline__ void mdq_step_tile(const MdqDesc &d, int64_t tl, int 
             }
         }
     } else {
-        // 17..32-bit codes: the reference's FP64 path verbatim.
+        // 17..32-bit codes: the reference's FP64 quotients, rounded and clamped, without an FP64
+        // division per element (mdq_code_f64).
         const double qlm = (double)d.qm;                        // 2^(bits-1), exact
         const double qlv = __builtin_ldexp(1.0, (int)d.bits) - 1.0;
+        const double ym = 1.0 / (double)dm, yv = 1.0 / (double)dv;
 #pragma unroll
         for (int e = 0; e < EPL; ++e) {
-            // a NaN quotient converts to 0 (the reference's (int) of NaN on its target)
-            double qm_ = __builtin_round((double)m[e] / (double)dm);
-            qm_ = qm_ == qm_ ? qm_ : 0.0;
-            qm_ = qm_ < -qlm ? -qlm : qm_;
-            qm_ = qm_ > qlm - 1.0 ? qlm - 1.0 : qm_;
-            double qv_ = __builtin_round((double)(lv[e] - s_vmin) / (double)dv);
-            qv_ = qv_ == qv_ ? qv_ : 0.0;
-            qv_ = qv_ < 0.0 ? 0.0 : qv_;
-            qv_ = qv_ > qlv ? qlv : qv_;
-            qmi[e] = (int32_t)qm_;
-            qvi[e] = (uint32_t)qv_;
+            const bool neg = f_bits(m[e]) >> 31;
+            const uint32_t k = mdq_code_f64(fabsf(m[e]), dm, ym, neg ? qlm : qlm - 1.0);
+            qmi[e] = (int32_t)(neg ? 0u - k : k);
+            qvi[e] = mdq_code_f64(lv[e] - s_vmin, dv, yv, qlv);
         }
     }
     if (prof_on) { unsigned long long t = clock64(); pa.c[3] += t - t0; t0 = t; }

@@ -152,6 +152,27 @@ MDQ_HD float mdq_round_half_away(float u, float d, float inv_lo, float hd)
     return R >= hd ? k0 + 1.0f : k0;
 }
 
+// min(round((double)u / (double)d), lim), ties away from zero, for floats u >= 0 and d >= 0 and
+// a whole lim in [0, 2^32); 0 where the quotient is no finite number (a NaN or infinite u or d),
+// as the reference's (int) of NaN on its target gives (stquant_kernel.cu:366,376).
+// y = RN(1 / d): q0 = RN(u y) is within 2^-51 of u / d, its residual r = u - q0 d is exact (a
+// multiple of the two operands' last places, below 2^26 of them), and q0 + r y lies within
+// 2^-104 of u / d.  The quotient of two 24-bit significands keeps 2^-78 away from every midpoint
+// of two doubles, so q = RN(q0 + r y) is the IEEE quotient.  floor(q + 1/2) is its rounding:
+// q + 1/2 is exact within q's binade, crossing into the next one cannot reach an integer that
+// q + 1/2 lies below, and q < 1/2 lies at least 2^-26 below.  Against one FP64 division and
+// round per code, 32-bit codes, B = 256, fp32 grads: GPT-2 small (HBM-bound) 589.5 -> 584.2 us,
+// 100 ragged tensors (163 MB, cache-resident) 34.8 -> 32.9 us, one tensor of 4,194,304 params
+// 22.3 -> 21.5 us; B = 64 and 1024 over GPT-2 small level.
+MDQ_HD uint32_t mdq_code_f64(float u, float d, double y, double lim)
+{
+    const double q0 = (double)u * y;
+    const double r = __builtin_fma(-q0, (double)d, (double)u);
+    const double q = __builtin_fma(r, y, q0);
+    // fmax drops a NaN
+    return (uint32_t)__builtin_fmin(__builtin_fmax(q + 0.5, 0.0), lim + 0.5);
+}
+
 // x / D correctly rounded for D = (float)(2^bits - 1), bits 1..32, given
 // y = RN(1/D): q = x*y is within an ulp, the fma residual x - q*D is exact,
 // and one correction q + r*y rounds to RN(x/D).  Checked against IEEE
