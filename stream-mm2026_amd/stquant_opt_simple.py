@@ -44,6 +44,7 @@ from __future__ import annotations
 import math
 import time
 from collections import Counter, OrderedDict
+from operator import itemgetter
 
 import numpy as np
 import torch
@@ -279,7 +280,8 @@ class MDQAdamWSimple(Optimizer):
         scored groups their width; fills the decision's timing keys."""
         dev = work[0][0].device
         lt = self.last_step_timings
-        steps = [self.state[p]["step"] for p, _g in work]
+        states = [self.state[p] for p, _g in work]
+        steps = [st["step"] for st in states]
         tau = self.param_groups[0]["tau"]
         self._settled = 0
         with _Stopwatch(dev) as sw:
@@ -297,7 +299,6 @@ class MDQAdamWSimple(Optimizer):
             # settling's decision stands where it changed no row and no other rank has a say
             scores, host, ema = made if mean is None else self._decision(stats, mean, steps, tau)
             self.n_ema, self.r_ema, self.v_global_ema = ema
-            states = [self.state[p] for p, _g in work]
             for (_p, g), st, s, h in zip(work, states, scores.unbind(0), host.tolist()):
                 st["last_score"] = s
                 if g.get("bits") is None:
@@ -422,6 +423,8 @@ class MDQAdamWSimple(Optimizer):
         hyper-parameters are refreshed.  Plans keep no reference to gradients.
         """
         buckets = OrderedDict()
+        launch_keys = {id(g): (min(int(g["block_size"]), 1024), mdq_hip.rounding_code(g.get("rounding", "nearest")),
+                               int(g.get("seed", 0) or 0)) for _p, g in items}
         for i, (p, group) in enumerate(items):
             state = self.state[p]
             grad = p.grad
@@ -430,9 +433,7 @@ class MDQAdamWSimple(Optimizer):
             if not grad.is_contiguous():
                 grad = grad.contiguous()
             ea, easq = state["exp_avg"], state["exp_avg_sq"]
-            key = (p.device, ea.dtype, easq.dtype, easq.numel() == 0, grad.dtype,
-                   min(int(group["block_size"]), 1024), mdq_hip.rounding_code(group.get("rounding", "nearest")),
-                   int(group.get("seed", 0) or 0))
+            key = (p.device, ea.dtype, easq.dtype, easq.numel() == 0, grad.dtype) + launch_keys[id(group)]
             buckets.setdefault(key, []).append((p, group, state, grad, i))
         cache = self.__dict__.setdefault("_plan_cache", {})
         runs = []
@@ -440,8 +441,8 @@ class MDQAdamWSimple(Optimizer):
             idx = [r[4] for r in rows]
             rows = [r[:4] for r in rows]
             dev, block, rnd, seed = key[0], key[5], key[6], key[7]
-            sig = tuple((id(p), p.data_ptr()) + tuple((id(st[k]), st[k].data_ptr()) for k in _STATE_TENSORS)
-                        for p, _g, st, _gr in rows)
+            tensors = [t for p, _g, st, _gr in rows for t in (p, *_state_tensors(st))]
+            sig = [*map(id, tensors)], [*map(torch.Tensor.data_ptr, tensors)]
             plan = cache.get(key)
             if plan is None or plan.sig != sig:
                 plan = self._plan_cls(self._entries(rows), block, rounding=rnd, seed=seed)
@@ -449,7 +450,7 @@ class MDQAdamWSimple(Optimizer):
                 # Strong references to the params and state tensors the plan points
                 # at: while they are held no other object can reuse their id(), so
                 # the id signature identifies exactly these tensors.
-                plan.keep = [(p,) + tuple(st[k] for k in _STATE_TENSORS) for p, _g, st, _gr in rows]
+                plan.keep = tensors
                 plan.sig = sig
                 cache[key] = plan
             else:
@@ -777,5 +778,5 @@ class MDQAdamWSimple(Optimizer):
         """Per-tensor bookkeeping a steady step skips (FusedIO counts fast-path tensors)."""
 
 
-_STATE_TENSORS = ("exp_avg", "exp_avg_sq", "scale_m", "scale_v", "v_min")
+_state_tensors = itemgetter("exp_avg", "exp_avg_sq", "scale_m", "scale_v", "v_min")
 _CODE_KEYS = ("exp_avg", "exp_avg_sq")
