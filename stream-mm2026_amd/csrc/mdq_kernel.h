@@ -1388,8 +1388,8 @@ __device__ __forceinline__ void mdq_step_tile_any(const MdqDesc &d, long long ti
     }
 }
 
-// Occupancy cap at 7 waves per SIMD in both kernels below: the clobber reserves v0..v71, so
-// the register file never holds 8 of these waves, whatever the compiler's count.  With one
+// Occupancy cap at 7 waves per SIMD at most in both kernels below: a clobber of v71 reserves
+// v0..v71, so the register file never holds 8 of these waves, whatever the compiler's count.  With one
 // contiguous eighth of the tiles per XCD, 8 waves ran the LLaMA 4-bit step 1 % slower
 // (same-allocation A/B 13.36 vs 13.23 ms); with the chunked tile order the two are level
 // (+-0.3 %).  Steps on int8 + uint8 codes, and with nearest rounding steps on packed 4-bit
@@ -1401,11 +1401,48 @@ __device__ __forceinline__ void mdq_step_tile_any(const MdqDesc &d, long long ti
 // the LLaMA-7B set 8 -> 16 -3.0 %, 4 -> 8 -1.9 %, 16 -> 4 -2.5 %, 16 -> 8 -0.7 %.  Packed
 // 4-bit codes with stochastic rounding keep 7 (6: LLaMA-7B +0.8 %, views B = 64 +1.2 %); most
 // other stochastic kernels need 73-85 VGPRs and hold 5-6 anyway.
-template <int SRC, int DST, bool SR>
+//
+// Steps on wider codes and at B = 1024 are capped by the bytes their waves ask for at once: a
+// wave issues all loads of its tile together, so W waves per SIMD keep W x 256 lanes x the lane's
+// load bytes (p, grads, codes) in flight per CU, and beyond about 104 KB more of them cost
+// bandwidth.  Measured on GPT-2 small, W = the compiler's own count -> the rule's:
+//   32-bit codes, fp32 grads (128 B a lane)   6 -> 3  601.2 -> 561.2 us at B = 128, 594.4 -> 564.1 at 256
+//   32-bit codes, bf16 grads (112 B)          6 -> 3  545.8 -> 524.4, 534.7 -> 517.2
+//   16-bit codes, fp32 grads (96 B)           5-7 -> 4  409.2 -> 396.1, 398.0 -> 390.8
+//   16-bit codes, bf16 grads (80 B)           5-7 -> 5  364.0 -> 360.6, 358.0 -> 358.0
+// At B = 1024 (twice the elements per lane) three waves are needed for their own arithmetic, and
+// more are too many: 4-bit 284.8 -> 275.8 (fp32 grads), 237.2 -> 232.4 (bf16), 8-bit 330.6 -> 316.4,
+// 279.8 -> 277.7, 16-bit 418.3 -> 403.8; two waves are slower (305.5, 281.1, 328.7, 325.7, 417.3)
+// except for 32-bit codes (224-256 B a lane): 622.1 -> 567.1, bf16 631.8 -> 551.8.
+// 8-bit codes with fp32 grads (80 B) as packed views, nearest rounding: 6 -> 5 waves 950.7 -> 929.8 us
+// (257 ragged tensors, B = 64), level otherwise.  As views 16-bit codes gain most (1418 -> 1320 us).
+// The one-tensor kernel (ONE) mostly runs on tensors that stay in cache, where 16-bit steps need the
+// waves for their arithmetic (4,194,304 params: 16.0 us, 16.2 by the rule): they keep the compiler's
+// count there, and 8-bit steps six waves.
+template <int SRC, int DST, int GT, int LOG2B, bool SR, bool VIEWS, bool ONE>
+constexpr int waves_per_simd()
+{
+    if (SRC == DST && ((SRC == ST_S16 && !ONE) || SRC == ST_S32 || LOG2B == 10)) {
+        constexpr int lane_bytes = Cfg<LOG2B>::EPL * (4 + (GT == GT_F32 ? 4 : 2) + code_size(SRC) * (SRC == ST_P4 ? 1 : 2));
+        constexpr int least = SRC == ST_S32 && LOG2B == 10 ? 2 : 3;
+        constexpr int w = 104 * 1024 / (256 * lane_bytes);
+        return w < least ? least : w > 7 ? 7 : w;
+    }
+    if (SRC == ST_S8 && DST == ST_S8) return VIEWS && !ONE && !SR && GT == GT_F32 ? 5 : 6;
+    return !SR && (SRC == ST_P4 || SRC != DST) ? 6 : 7;
+}
+
+// Reserves registers up to the count that leaves room for waves_per_simd waves.
+template <int W>
 __device__ __forceinline__ void occupancy_cap()
 {
-    if constexpr ((SRC == ST_S8 && DST == ST_S8) || (!SR && (SRC == ST_P4 || SRC != DST))) asm volatile("" ::: "v79");
-    else asm volatile("" ::: "v71");
+    static_assert(W >= 2 && W <= 7, "register counts below");
+    if constexpr (W == 7) asm volatile("" ::: "v71");
+    else if constexpr (W == 6) asm volatile("" ::: "v79");
+    else if constexpr (W == 5) asm volatile("" ::: "v95");
+    else if constexpr (W == 4) asm volatile("" ::: "v127");
+    else if constexpr (W == 3) asm volatile("" ::: "v135");
+    else asm volatile("" ::: "v175");
 }
 
 // The launch over a descriptor table: the tile's tensor is the largest t with
@@ -1418,7 +1455,7 @@ __global__ __launch_bounds__(Cfg<LOG2B>::THREADS) void mdq_step_kernel(const Mdq
                                                                       unsigned long long *__restrict__ prof,
                                                                       const StepArgs sa)
 {
-    occupancy_cap<SRC, DST, SR>();
+    occupancy_cap<waves_per_simd<SRC, DST, GT, LOG2B, SR, VIEWS, false>()>();
     using L = StepLds<SRC, DST, GT, LOG2B, SR, VIEWS>;
     __shared__ float lut_s[L::LUT];
     __shared__ int32_t xw_s[6];
@@ -1444,7 +1481,7 @@ __global__ __launch_bounds__(Cfg<LOG2B>::THREADS) void mdq_step_kernel_one(const
                                                                           unsigned long long *__restrict__ prof,
                                                                           const StepArgs sa)
 {
-    occupancy_cap<SRC, SRC, SR>();
+    occupancy_cap<waves_per_simd<SRC, SRC, GT, LOG2B, SR, true, true>()>();
     using L = StepLds<SRC, SRC, GT, LOG2B, SR, true>;
     __shared__ float lut_s[L::LUT];
     __shared__ int32_t xw_s[6];
