@@ -1393,12 +1393,11 @@ __device__ __forceinline__ void mdq_step_tile_any(const MdqDesc &d, long long ti
 // contiguous eighth of the tiles per XCD, 8 waves ran the LLaMA 4-bit step 1 % slower
 // (same-allocation A/B 13.36 vs 13.23 ms); with the chunked tile order the two are level
 // (+-0.3 %).  Steps on int8 + uint8 codes, and with nearest rounding steps on packed 4-bit
-// codes and storage-changing steps, are capped at 6 (v0..v79 reserved): their waves spend most
+// codes, are capped at 6 (v0..v79 reserved): their waves spend most
 // of a tile waiting for its loads, and one wave fewer per SIMD contends less.  Same-allocation
 // A/B, nearest rounding: 8-bit config 5 B = 64 / 128 / 256 -2.0 / -1.9 / -1.3 %, as packed views
 // B = 128 -1.6 %, LLaMA-7B -0.7 %; 4-bit (three boxes) LLaMA-7B -0.3 to -0.6 %, GPT-2 small
-// -0.3 %, config 5 B = 64 -1.0 %, as packed views B = 128 -2.2 to -2.7 %; storage changes on
-// the LLaMA-7B set 8 -> 16 -3.0 %, 4 -> 8 -1.9 %, 16 -> 4 -2.5 %, 16 -> 8 -0.7 %.  Packed
+// -0.3 %, config 5 B = 64 -1.0 %, as packed views B = 128 -2.2 to -2.7 %.  Packed
 // 4-bit codes with stochastic rounding keep 7 (6: LLaMA-7B +0.8 %, views B = 64 +1.2 %); most
 // other stochastic kernels need 73-85 VGPRs and hold 5-6 anyway.
 //
@@ -1419,17 +1418,23 @@ __device__ __forceinline__ void mdq_step_tile_any(const MdqDesc &d, long long ti
 // The one-tensor kernel (ONE) mostly runs on tensors that stay in cache, where 16-bit steps need the
 // waves for their arithmetic (4,194,304 params: 16.0 us, 16.2 by the rule): they keep the compiler's
 // count there, and 8-bit steps six waves.
+// Storage-changing steps follow the same rule with the wider side's codes, between 3 and 5 waves
+// (6 and 7 before): one LLaMA-7B layer, B = 128, nearest: 16 -> 4 fp32 grads 568 -> 548 us, 8 -> 16 589 ->
+// 580, 32 -> 16 832 -> 775, bf16 grads 32 -> 4 640 -> 621, 8 -> 4 420 -> 415; 16 -> 4 and back with
+// bf16 grads, B = 256: 483.4 -> 478.9 a step.
 template <int SRC, int DST, int GT, int LOG2B, bool SR, bool VIEWS, bool ONE>
 constexpr int waves_per_simd()
 {
-    if (SRC == DST && ((SRC == ST_S16 && !ONE) || SRC == ST_S32 || LOG2B == 10)) {
-        constexpr int lane_bytes = Cfg<LOG2B>::EPL * (4 + (GT == GT_F32 ? 4 : 2) + code_size(SRC) * (SRC == ST_P4 ? 1 : 2));
+    constexpr auto code_bytes = [](int st) { return code_size(st) * (st == ST_P4 ? 1 : 2); };
+    constexpr int codes = code_bytes(SRC) > code_bytes(DST) ? code_bytes(SRC) : code_bytes(DST);
+    constexpr int w = 104 * 1024 / (256 * Cfg<LOG2B>::EPL * (4 + (GT == GT_F32 ? 4 : 2) + codes));
+    if (SRC != DST) return w < 3 ? 3 : w > 5 ? 5 : w;
+    if ((SRC == ST_S16 && !ONE) || SRC == ST_S32 || LOG2B == 10) {
         constexpr int least = SRC == ST_S32 && LOG2B == 10 ? 2 : 3;
-        constexpr int w = 104 * 1024 / (256 * lane_bytes);
         return w < least ? least : w > 7 ? 7 : w;
     }
-    if (SRC == ST_S8 && DST == ST_S8) return VIEWS && !ONE && !SR && GT == GT_F32 ? 5 : 6;
-    return !SR && (SRC == ST_P4 || SRC != DST) ? 6 : 7;
+    if (SRC == ST_S8) return VIEWS && !ONE && !SR && GT == GT_F32 ? 5 : 6;
+    return !SR && SRC == ST_P4 ? 6 : 7;
 }
 
 // Reserves registers up to the count that leaves room for waves_per_simd waves.
