@@ -751,6 +751,7 @@ int run_convert(const stq_code_convert *items, int n, hipStream_t stream)
     std::vector<mdq::ConvDesc> d;
     d.reserve((size_t)n);
     int64_t tiles = 0;
+    bool wide = true;      // every tensor has 4-byte codes on one side
     for (int i = 0; i < n; ++i) {
         const stq_code_convert &c = items[i];
         if (c.numel < 0) return fail(STQ_ERR_INVALID, "tensor %d: negative numel", i);
@@ -770,6 +771,7 @@ int run_convert(const stq_code_convert *items, int n, hipStream_t stream)
         e.tile_begin = tiles;
         e.src = c.src_storage;
         e.dst = c.dst_storage;
+        wide = wide && (c.src_storage == STQ_STORE_S32 || c.dst_storage == STQ_STORE_S32);
         tiles += (c.numel + mdq::CONV_TILE - 1) / mdq::CONV_TILE;
         d.push_back(e);
     }
@@ -795,7 +797,7 @@ int run_convert(const stq_code_convert *items, int n, hipStream_t stream)
     hipError_t e;
     e = mdq::launch_convert(reinterpret_cast<const mdq::ConvDesc *>(s->dev),
                             reinterpret_cast<const long long *>(s->dev + m * sizeof(mdq::ConvDesc)), (int)m,
-                            tiles, stream);
+                            tiles, wide, stream);
     if (e != hipSuccess) return hip_fail(e, "convert launch");
     return release_slot(s, stream);
 }

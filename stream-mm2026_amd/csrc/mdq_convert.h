@@ -24,6 +24,8 @@ struct alignas(16) ConvDesc {
 
 static_assert(sizeof(ConvDesc) == 64, "ConvDesc layout");
 
-hipError_t launch_convert(const ConvDesc *d, const long long *tile_begin, int n, long long tiles, hipStream_t s);
+// wide: every tensor has ST_S32 codes on one side.
+hipError_t launch_convert(const ConvDesc *d, const long long *tile_begin, int n, long long tiles, bool wide,
+                          hipStream_t s);
 
 }  // namespace mdq

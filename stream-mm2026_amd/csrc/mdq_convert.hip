@@ -214,8 +214,125 @@ __device__ __forceinline__ void tile_vec_src(const ConvDesc &t, int64_t base)
     }
 }
 
+// 4 codes of one array, W = code_size dwords.
+template <int W> struct Words { typedef uint32_t T; };
+template <> struct Words<2> { typedef cu2 T; };
+template <> struct Words<4> { typedef cu4 T; };
+
+// The 4 codes at element i, as loaded and as values.
+template <int ST> struct Raw4 {
+    typedef typename Words<code_size<ST>()>::T T;
+    T m, v;
+};
+
+template <int ST>
+__device__ __forceinline__ Raw4<ST> load4(const ConvDesc &t, int64_t i)
+{
+    typedef typename Raw4<ST>::T T;
+    constexpr int cs = code_size<ST>();
+    Raw4<ST> r{};
+    r.m = ldv<T>(static_cast<const char *>(t.src_m) + i * cs);
+    if constexpr (ST != ST_P4) r.v = ldv<T>(static_cast<const char *>(t.src_v) + i * cs);
+    return r;
+}
+
+template <int ST>
+__device__ __forceinline__ void unpack4(const Raw4<ST> &r, int32_t (&m)[4], uint32_t (&v)[4])
+{
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        if constexpr (ST == ST_P4) {
+            m[k] = (int32_t)((r.m >> (8 * k)) & 15u) - 8;
+            v[k] = (r.m >> (8 * k + 4)) & 15u;
+        } else if constexpr (ST == ST_S8) {
+            m[k] = (int32_t)(int8_t)(r.m >> (8 * k));
+            v[k] = (r.v >> (8 * k)) & 0xffu;
+        } else if constexpr (ST == ST_S16) {
+            m[k] = (int32_t)(int16_t)(r.m[k >> 1] >> (16 * (k & 1)));
+            v[k] = (r.v[k >> 1] >> (16 * (k & 1))) & 0xffffu;
+        } else {
+            m[k] = (int32_t)r.m[k];
+            v[k] = r.v[k];
+        }
+    }
+}
+
+// store8 for 4 codes.
+template <int ST>
+__device__ __forceinline__ void store4(const ConvDesc &t, int64_t i, const int32_t (&m)[4], const uint32_t (&v)[4])
+{
+    constexpr int cs = code_size<ST>();
+    char *pm = static_cast<char *>(t.dst_m) + i * cs;
+    char *pv = static_cast<char *>(t.dst_v) + i * cs;
+    if constexpr (ST == ST_S32) {
+        stv<cu4>(cu4{(uint32_t)m[0], (uint32_t)m[1], (uint32_t)m[2], (uint32_t)m[3]}, pm);
+        stv<cu4>(cu4{v[0], v[1], v[2], v[3]}, pv);
+    } else if constexpr (ST == ST_S16) {
+        uint32_t a[4], b[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            a[k] = (uint32_t)clampi(m[k], -32768, 32767) & 0xffffu;
+            b[k] = minu(v[k], 65535u);
+        }
+        stv<cu2>(cu2{a[0] | (a[1] << 16), a[2] | (a[3] << 16)}, pm);
+        stv<cu2>(cu2{b[0] | (b[1] << 16), b[2] | (b[3] << 16)}, pv);
+    } else {
+        uint32_t wm = 0u, wv = 0u;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if constexpr (ST == ST_P4) {
+                wm |= ((uint32_t)(clampi(m[k], -8, 7) + 8) | (minu(v[k], 15u) << 4)) << (8 * k);
+            } else {
+                wm |= ((uint32_t)clampi(m[k], -128, 127) & 0xffu) << (8 * k);
+                wv |= minu(v[k], 255u) << (8 * k);
+            }
+        }
+        stv<uint32_t>(wm, pm);
+        if constexpr (ST == ST_S8) stv<uint32_t>(wv, pv);
+    }
+}
+
+// One whole tile of a pair with 4-byte codes, 4 elements at a time.  The codes stay as loaded
+// until they are stored: unpacked they would take the kernel from 8 waves per SIMD to 5.
+template <int SRC, int DST>
+__device__ __forceinline__ void tile_vec4(const ConvDesc &t, int64_t base)
+{
+    constexpr int ITERS = CONV_TILE / (4 * CV_THREADS);
+    static_assert(ITERS * CV_THREADS * 4 == CONV_TILE, "tile = threads x 4 x iterations");
+    Raw4<SRC> r[ITERS];
+#pragma unroll
+    for (int k = 0; k < ITERS; ++k) r[k] = load4<SRC>(t, base + (int64_t)(k * CV_THREADS + (int)threadIdx.x) * 4);
+#pragma unroll
+    for (int k = 0; k < ITERS; ++k) {
+        int32_t m[4];
+        uint32_t v[4];
+        unpack4<SRC>(r[k], m, v);
+        store4<DST>(t, base + (int64_t)(k * CV_THREADS + (int)threadIdx.x) * 4, m, v);
+    }
+}
+
+// The same for a pair known at run time, one side of which has 4-byte codes.
+__device__ __forceinline__ void tile_vec4_any(const ConvDesc &t, int64_t base)
+{
+    switch (t.src * 4 + t.dst) {
+    case ST_P4 * 4 + ST_S32: tile_vec4<ST_P4, ST_S32>(t, base); break;
+    case ST_S8 * 4 + ST_S32: tile_vec4<ST_S8, ST_S32>(t, base); break;
+    case ST_S16 * 4 + ST_S32: tile_vec4<ST_S16, ST_S32>(t, base); break;
+    case ST_S32 * 4 + ST_P4: tile_vec4<ST_S32, ST_P4>(t, base); break;
+    case ST_S32 * 4 + ST_S8: tile_vec4<ST_S32, ST_S8>(t, base); break;
+    case ST_S32 * 4 + ST_S16: tile_vec4<ST_S32, ST_S16>(t, base); break;
+    default: tile_vec4<ST_S32, ST_S32>(t, base); break;
+    }
+}
+
 __device__ __forceinline__ bool al16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// WIDE: every tensor of the launch has 4-byte codes on one side.  Its tiles move 4 elements at a
+// time, one 16-byte access per array of those codes: with 8, as two accesses 32 bytes apart, each
+// store instruction wrote half of every line it touched (one LLaMA-7B layer, nibbles to int32
+// 594 -> 365 us, int16 to int32 521 -> 446, int32 to int16 420 -> 405).  An instance of its own: with both
+// tile forms in one kernel the narrow pairs ran 2 to 8 % slower.
+template <bool WIDE>
 __global__ __launch_bounds__(CV_THREADS) void convert_kernel(const ConvDesc *__restrict__ d, int n,
                                                              const long long *__restrict__ tb)
 {
@@ -231,6 +348,10 @@ __global__ __launch_bounds__(CV_THREADS) void convert_kernel(const ConvDesc *__r
     const bool vec = base + CONV_TILE <= t.numel && al16(t.src_m) && al16(t.dst_m) &&
                      (t.src == ST_P4 || al16(t.src_v)) && (t.dst == ST_P4 || al16(t.dst_v));
     if (vec) {
+        if constexpr (WIDE) {
+            tile_vec4_any(t, base);
+            return;
+        }
         switch (t.src) {
         case ST_P4: tile_vec_src<ST_P4>(t, base); break;
         case ST_S8: tile_vec_src<ST_S8>(t, base); break;
@@ -251,10 +372,12 @@ __global__ __launch_bounds__(CV_THREADS) void convert_kernel(const ConvDesc *__r
 
 }  // namespace
 
-hipError_t launch_convert(const ConvDesc *d, const long long *tile_begin, int n, long long tiles, hipStream_t s)
+hipError_t launch_convert(const ConvDesc *d, const long long *tile_begin, int n, long long tiles, bool wide,
+                          hipStream_t s)
 {
     if (n <= 0 || tiles <= 0) return hipSuccess;
-    convert_kernel<<<dim3((unsigned)tiles), dim3(CV_THREADS), 0, s>>>(d, n, tile_begin);
+    if (wide) convert_kernel<true><<<dim3((unsigned)tiles), dim3(CV_THREADS), 0, s>>>(d, n, tile_begin);
+    else convert_kernel<false><<<dim3((unsigned)tiles), dim3(CV_THREADS), 0, s>>>(d, n, tile_begin);
     return hipGetLastError();
 }
 

@@ -175,3 +175,28 @@ def test_every_storage_pair_matches_the_value_map(src, dst):
         else:
             assert np.array_equal(as_i64(nm.cpu()).numpy(), w[0]), f"m codes, n={n}"
             assert np.array_equal(as_i64(nv.cpu()).numpy(), w[1]), f"v codes, n={n}"
+
+
+@pytest.mark.parametrize("pairs", [[("p4", "s32"), ("s32", "s16"), ("s32", "p4")], [("p4", "s32"), ("s8", "s16"), ("s32", "s8")]])
+def test_launches_with_and_without_a_narrow_pair(pairs):
+    """Several storage pairs in one launch: all with 4-byte codes on one side (the instance that moves 4
+    elements per access), and with a pair that has none (the instance that moves 8)."""
+    print(f"case: convert pairs {pairs}", flush=True)
+    items, want = [], []
+    for k, (src, dst) in enumerate(pairs):
+        for n in (4095, 4096, 8192 + 3):
+            cm, cv = rand_codes(src, n, 71 * k + n)
+            m, v = _decode(src, cm, cv)
+            (mlo, mhi), (vlo, vhi) = _RANGE[dst]
+            m, v = np.clip(m, mlo, mhi), np.clip(v, vlo, vhi)
+            want.append((m + 8) | (v << 4) if dst == "p4" else (m, v))
+            gm = cm.to(DEV)
+            items.append((gm, cv.to(DEV)) + tuple(mdq_hip.empty_codes(gm, _STORE[dst])))
+    mdq_hip.convert_codes(items)
+    torch.cuda.synchronize()
+    for (_sm, _sv, nm, nv), w in zip(items, want):
+        if nv.numel() == 0:
+            assert np.array_equal(nm.cpu().numpy().astype(np.int64), w)
+        else:
+            assert np.array_equal(as_i64(nm.cpu()).numpy(), w[0])
+            assert np.array_equal(as_i64(nv.cpu()).numpy(), w[1])
