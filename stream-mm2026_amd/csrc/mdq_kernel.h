@@ -1431,7 +1431,7 @@ __device__ __forceinline__ void mdq_step_tile_any(const MdqDesc &d, long long ti
 // Storage-changing steps follow the same rule with the wider side's codes, between 3 and 5 waves
 // (6 and 7 before): one LLaMA-7B layer, B = 128, nearest: 16 -> 4 fp32 grads 568 -> 548 us, 8 -> 16 589 ->
 // 580, 32 -> 16 832 -> 775, bf16 grads 32 -> 4 640 -> 621, 8 -> 4 420 -> 415; 16 -> 4 and back with
-// bf16 grads, B = 256: level to -1 % (box to box).
+// bf16 grads, B = 256: level to -1 % (run to run).
 template <int SRC, int DST, int GT, int LOG2B, bool SR, bool VIEWS, bool ONE>
 constexpr int waves_per_simd()
 {
