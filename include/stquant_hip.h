@@ -183,11 +183,14 @@ int stq_multi_tensor_mdq_adamw_noalloc(const stq_tensor *tensors, int n_tensors,
  *   stats[3i + 1] = std(g) / (mean(|g|) + 1e-12)   (std unbiased; NaN if numel == 1),
  *   stats[3i + 2] = mean(g^2)                       (NaN means if numel == 0),
  * into the device array stats[3 * n_tensors].  Sums are accumulated in fp64 in
- * a fixed order (deterministic); the final divisions, square roots and the
- * 1e-12 add are fp32, as the reference's.  Differs from the reference's fp32
+ * a fixed order (deterministic; whole 32768-element tiles of a tensor that starts
+ * on 16 bytes sum each 16 bytes' values in fp32 first); the final divisions,
+ * square roots and the 1e-12 add are fp32, as the reference's.  A grad may start
+ * at any byte address; apart from whether it is a multiple of 16, the address does
+ * not change the result.  Differs from the reference's fp32
  * torch reductions by rounding only (about 1e-7 relative).  grads and numels
  * are host arrays; the library keeps the descriptor table and the partial
- * sums (24 bytes per 32768 elements) in its per-device ring.
+ * sums (32 bytes per 32768 elements) in its per-device ring.
  *
  * Replaces MDQAdamWSimple._compute_grad_stats called once per tensor
  * (/root/reference/CUDA/stquant_opt_simple.py:93-98, loop at :427-431).

@@ -534,12 +534,11 @@ int run_grad_stats(const void *const *grads, const int64_t *numels, int n, int g
     if (n == 0) return STQ_OK;
     std::vector<mdq::StatDesc> d((size_t)n);
     int64_t tiles = 0;
+    bool off16 = false;
     for (int i = 0; i < n; ++i) {
         if (numels[i] < 0) return fail(STQ_ERR_INVALID, "tensor %d: negative numel", i);
         if (numels[i] > 0 && !grads[i]) return fail(STQ_ERR_INVALID, "tensor %d: null grad", i);
-        // the kernel finds a tensor's place in its first line by element counts
-        if (numels[i] > 0 && !is_aligned(grads[i], grad_dt == STQ_FLOAT ? 4 : 2))
-            return fail(STQ_ERR_INVALID, "tensor %d: grad must be aligned to its element size", i);
+        off16 = off16 || (numels[i] >= mdq::STAT_TILE && !is_aligned(grads[i], 16));
         d[i].g = grads[i];
         d[i].numel = numels[i];
         d[i].tile_begin = tiles;
@@ -568,7 +567,7 @@ int run_grad_stats(const void *const *grads, const int64_t *numels, int n, int g
     const mdq::StatDesc *dd = reinterpret_cast<const mdq::StatDesc *>(s->dev);
     const long long *dtb = reinterpret_cast<const long long *>(s->dev + (size_t)n * sizeof(mdq::StatDesc));
     double *partials = reinterpret_cast<double *>(s->dev + part_off);
-    e = mdq::launch_grad_stats(dd, dtb, n, tiles, grad_dt, partials, stats, stream);
+    e = mdq::launch_grad_stats(dd, dtb, n, tiles, grad_dt, off16, partials, stats, stream);
     if (e != hipSuccess) return hip_fail(e, "grad_stats launch");
     return release_slot(s, stream);
 }

@@ -22,9 +22,10 @@ struct alignas(16) StatDesc {
 static_assert(sizeof(StatDesc) == 32, "StatDesc layout");
 
 // partials: 4 doubles per tile (sum g, sum of squared deviations from the tile
-// mean, sum g^2, sum |g|); out: 3 floats per tensor (n_l, r_l, v_l).
+// mean, sum g^2, sum |g|); out: 3 floats per tensor (n_l, r_l, v_l).  off16: some tensor of at
+// least STAT_TILE elements does not start on a multiple of 16 bytes.
 hipError_t launch_grad_stats(const StatDesc *d, const long long *tile_begin, int n, long long tiles,
-                             int grad_dt, double *partials, float *out, hipStream_t s);
+                             int grad_dt, bool off16, double *partials, float *out, hipStream_t s);
 
 // The bit decision's scores of n > 0 tensors from their statistics stats[3n] and the mean of
 // those over the tensors: out[0 .. n) the scores, out[n .. 2n) the r_l; ema[3] the EMAs

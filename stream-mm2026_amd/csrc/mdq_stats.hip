@@ -17,14 +17,14 @@
 //      mean, and non-finite or tiny (squares below fp32's normal range) values are
 //      redone in fp64.  The threads' (mean, M2) then merge pairwise by Chan's
 //      formula for equal counts, across lanes and across the workgroup's waves.
-//      A whole tile takes this path at any element offset (a view of a flat grad
-//      buffer): its pieces are read from its 128-byte line on and the first 8 threads
-//      trade the bytes in front of it for those behind the last whole piece.  A ragged
-//      last tile takes masked pieces, per-element fp64 sums and a second pass for the
-//      deviations from its mean.  Before, both kinds were read element by element, 64
-//      dependent loads a thread and pass: 257 ragged bf16 tensors packed back to back
-//      (363,174,740 elements, 726 MB) 689 -> 124 us a call, the kernel 675 -> 110 us
-//      (6.6 TB/s).  The errors against 64 bits did not change (the final fp32 rounding).
+//      A ragged last tile, and every tile of a tensor that does not start on 16 bytes (a
+//      view of a flat grad buffer), takes per-element fp64 sums and a second pass for the
+//      deviations from its mean: thread i sums the elements i, i + 512, ... in that order,
+//      so the bits do not depend on where in its line the tensor starts (tile_f64).  About
+//      twenty lane operations an element, twelve of them fp64 or conversions: 16-bit views
+//      are VALU-bound there (257 ragged bf16 tensors packed back to back, 726 MB: 184 us a
+//      call, 119 on 16-byte boundaries), fp32 views near the memory's rate (1453 MB: 234 us).
+//      Loaded one element at a time, each waited for, they took 700 and 732 us.
 //   2. stats_finish_kernel: one workgroup per tensor combines its tiles in a fixed
 //      order.  The squared deviations combine by Chan's pairwise formula,
 //      M2 = sum M2_i + sum n_i (mean_i - mean)^2, which stays accurate however
@@ -33,7 +33,8 @@
 //      inf, as the reference's fp32 accumulators overflow.
 //   3. scores_kernel (a call of its own, after the caller's mean over the tensors):
 //      one thread per tensor folds the mean into the EMAs and forms the tensor's score.
-// Both orders are fixed by the tensor list, so results are deterministic.
+// Both orders are fixed by the tensors' sizes and by whether each starts on 16 bytes, so results
+// are deterministic and do not depend on the addresses otherwise.
 #include <hip/hip_runtime.h>
 
 #include "mdq_desc.h"
@@ -54,12 +55,17 @@ __device__ __forceinline__ float f16_to_f(uint32_t h) { return (float)__builtin_
 // wait for all together.
 #define ST_GLOBAL __attribute__((address_space(1)))
 
+// Element e of a grad at any byte address: the element types below ask for no alignment, which
+// costs nothing (a load of 2 or 4 bytes is one instruction at any address on this target).
+typedef float any_f32 __attribute__((aligned(1)));
+typedef unsigned short any_u16 __attribute__((aligned(1)));
+
 template <int GT>
 __device__ __forceinline__ float load_one(const void *g, int64_t e)
 {
-    if constexpr (GT == GT_F32) return ((const ST_GLOBAL float *)g)[e];
-    else if constexpr (GT == GT_BF16) return bf16_to_f(((const ST_GLOBAL unsigned short *)g)[e]);
-    else return f16_to_f(((const ST_GLOBAL unsigned short *)g)[e]);
+    if constexpr (GT == GT_F32) return ((const ST_GLOBAL any_f32 *)g)[e];
+    else if constexpr (GT == GT_BF16) return bf16_to_f(((const ST_GLOBAL any_u16 *)g)[e]);
+    else return f16_to_f(((const ST_GLOBAL any_u16 *)g)[e]);
 }
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -68,23 +74,13 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // Elements per 16-byte load.
 template <int GT> constexpr int vec_elems() { return GT == GT_F32 ? 4 : 8; }
 
-// The 16-byte piece w of a line (non-temporal), kept as loaded (16-bit grads take half the
-// registers of their fp32 values).
-__device__ __forceinline__ u32x4 load_piece(const char *line, int w)
+// One 16-byte non-temporal load at element e (16-byte aligned), kept as loaded
+// (16-bit grads take half the registers of their fp32 values).
+template <int GT>
+__device__ __forceinline__ u32x4 load_raw(const void *g, int64_t e)
 {
-    return __builtin_nontemporal_load((const ST_GLOBAL u32x4 *)(line + 16 * (int64_t)w));
-}
-
-// The first nb bytes of a (nb > 0, even; all of it from 16 on), the rest of b.
-__device__ __forceinline__ u32x4 splice(const u32x4 a, const u32x4 b, uint32_t nb)
-{
-    u32x4 r;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t m = nb >= 4u * i + 4u ? 0xffffffffu : (nb <= 4u * i ? 0u : 0xffffu);
-        r[i] = (a[i] & m) | (b[i] & ~m);
-    }
-    return r;
+    constexpr int ES = GT == GT_F32 ? 4 : 2;   // bytes per element
+    return __builtin_nontemporal_load((const ST_GLOBAL u32x4 *)(static_cast<const char *>(g) + ES * e));
 }
 
 // The fp32 values of one loaded 16-byte vector.
@@ -156,7 +152,101 @@ __device__ __forceinline__ void block_sum(double (&v)[K], double (*lds)[K])
     __syncthreads();   // lds is free for the next block_sum
 }
 
+// The partial sums of a tile of cnt elements from per-element fp64 sums: the tile mean, then the
+// squared deviations from it.  each(f) calls f(value, whether it is one of the tile's) for this
+// thread's elements i, i + 512, ... in that order.
+template <class Each>
+__device__ __forceinline__ void tile_f64(uint32_t cnt, Each each, double *__restrict__ partial, double (*lds3)[3],
+                                         double (*lds2)[2])
+{
+    double s[3] = {0.0, 0.0, 0.0};      // sum g, sum g^2, sum |g|
+    each([&](float x, bool in) { acc(s[0], s[1], s[2], in ? x : 0.0f); });
+    block_sum<3>(s, lds3);
+    const double n_t = (double)cnt;
+    const float c = (float)(s[0] / n_t);
+    double dv[2] = {0.0, 0.0};          // sum d, sum d^2 with d = g - c
+    each([&](float x, bool in) {
+        const double dd = in ? (double)x - (double)c : 0.0;
+        dv[0] += dd;
+        dv[1] = fma(dd, dd, dv[1]);
+    });
+    block_sum<2>(dv, lds2);
+    if (threadIdx.x == 0) {
+        // d = g - c is exact in fp64, so M2 = sum d^2 - (sum d)^2 / n and sum g = n c + sum d
+        // are as accurate as the tile's spread allows (non-finite g: the first pass's sum)
+        partial[0] = fabs(dv[0]) <= __DBL_MAX__ ? fma(n_t, (double)c, dv[0]) : s[0];
+        partial[1] = dv[1] - dv[0] * (dv[0] / n_t);
+        partial[2] = s[1];
+        partial[3] = s[2];
+    }
+}
+
+// A whole tile at any byte address.  Each thread keeps its elements from the first pass for the
+// second (a 16-bit pair in one register), 113 registers in fp32 and 92 in 16 bits; read again
+// instead, 8 in flight as for a ragged tile, the 257 ragged tensors take 350 us in place of 234 in
+// fp32 and 227 in place of 184 in bf16.  16 loads at a time: 32 and 64 take 196 and 203 us in bf16.
 template <int GT>
+__device__ __forceinline__ void whole_f64(const void *g, double *__restrict__ partial, double (*lds3)[3],
+                                          double (*lds2)[2])
+{
+    constexpr int NE = STAT_TILE / ST_THREADS;     // elements per thread
+    constexpr int P = GT == GT_F32 ? 1 : 2;        // elements per register
+    constexpr int G = 16;                          // loaded together
+    uint32_t raw[NE / P];
+#pragma unroll
+    for (int k0 = 0; k0 < NE; k0 += G) {
+        uint32_t w[G];
+#pragma unroll
+        for (int k = 0; k < G; ++k) {
+            const uint32_t i = (uint32_t)((k0 + k) * ST_THREADS) + threadIdx.x;
+            if constexpr (P == 1) w[k] = __float_as_uint(((const ST_GLOBAL any_f32 *)g)[i]);
+            else w[k] = ((const ST_GLOBAL any_u16 *)g)[i];
+        }
+#pragma unroll
+        for (int k = 0; k < G; k += P) raw[(k0 + k) / P] = P == 1 ? w[k] : w[k] | (w[k + P - 1] << 16);
+    }
+    tile_f64((uint32_t)STAT_TILE, [&](auto &&f) {
+#pragma unroll
+        for (int r = 0; r < NE / P; ++r) {
+            // opaque in each pass: the compiler would keep every element's fp64 value from the
+            // first one, 128 registers, instead of widening it again
+            asm volatile("" : "+v"(raw[r]));
+            if constexpr (GT == GT_F32) {
+                f(__uint_as_float(raw[r]), true);
+            } else {
+                f(GT == GT_BF16 ? bf16_to_f(raw[r] & 0xffffu) : f16_to_f(raw[r] & 0xffffu), true);
+                f(GT == GT_BF16 ? bf16_to_f(raw[r] >> 16) : f16_to_f(raw[r] >> 16), true);
+            }
+        }
+    }, partial, lds3, lds2);
+}
+
+// A ragged last tile of cnt elements at any byte address, read once a pass (the second time from
+// L2) with 8 loads a thread in flight: 16 take the kernel from 6 waves per SIMD to 5.
+template <int GT>
+__device__ __forceinline__ void ragged_f64(const void *g, uint32_t cnt, double *__restrict__ partial, double (*lds3)[3],
+                                           double (*lds2)[2])
+{
+    constexpr int G = 8;
+    tile_f64(cnt, [&](auto &&f) {
+#pragma unroll 1
+        for (uint32_t i0 = threadIdx.x; i0 < cnt; i0 += G * ST_THREADS) {
+            float x[G];
+#pragma unroll
+            for (int k = 0; k < G; ++k) {
+                const uint32_t i = i0 + (uint32_t)(k * ST_THREADS);
+                x[k] = load_one<GT>(g, i < cnt ? i : cnt - 1u);
+            }
+#pragma unroll
+            for (int k = 0; k < G; ++k) f(x[k], i0 + (uint32_t)(k * ST_THREADS) < cnt);
+        }
+    }, partial, lds3, lds2);
+}
+
+// OFF16: some tensor of the launch starts off 16 bytes and has a whole tile.  An instance of its
+// own: whole_f64's registers would leave the 16-byte path 4 waves per SIMD (257 aligned ragged
+// bf16 tensors 119 -> 135 us).
+template <int GT, bool OFF16>
 __global__ __launch_bounds__(ST_THREADS) void stats_partial_kernel(const StatDesc *__restrict__ d, int n,
                                                                    const long long *__restrict__ tb,
                                                                    double *__restrict__ partials)
@@ -182,40 +272,18 @@ __global__ __launch_bounds__(ST_THREADS) void stats_partial_kernel(const StatDes
     }
     const StatDesc t = d[lo];
     const int64_t base = (tile - t.tile_begin) * STAT_TILE;
-    // (formed from two sums: the compiler lowered cnt = min(numel - base, STAT_TILE) == STAT_TILE
-    // to a select on a stale condition bit)
-    const bool whole = base + STAT_TILE <= t.numel;
-    constexpr int V = vec_elems<GT>();
-    constexpr int ES = 16 / V;                     // bytes per element
-    constexpr int NL = STAT_TILE / (V * ST_THREADS);
-    // The tile's first byte, its 128-byte line and its offset in it, in bytes and elements.
-    // Both paths read whole aligned 16-byte pieces counted from that line: piece w holds the
-    // elements V w - offe .. V w - offe + V - 1 of the tile.  A piece is read only if it
-    // holds an element of the tile, so the bytes around the tensor that it carries lie on
-    // pages that the tensor maps.
-    const char *g0 = static_cast<const char *>(t.g) + base * ES;
-    const uint32_t off = (uint32_t)reinterpret_cast<uintptr_t>(g0) & 127u;
-    const char *line = g0 - off;
-    const int offe = (int)(off / ES);
-    if (whole) {
-        // A whole tile at any element offset, one pass: each thread loads STAT_TILE /
-        // ST_THREADS elements and sums x, x^2 and |x| (fp32 over each loaded piece,
-        // pairwise; fp64 across pieces).  A tile that starts inside its line has off more
-        // bytes in front than pieces 0 .. STAT_TILE / V - 1 cover, and its last off bytes
-        // lie in the pieces behind them; the bytes in front of the tile that the first 8
-        // threads hold are replaced by those, so every thread has its STAT_TILE / ST_THREADS
-        // elements and the sums below run as for an aligned tile.
+    const int64_t left = t.numel - base;           // elements from the tile's first one on
+    if (left >= STAT_TILE && (!OFF16 || (reinterpret_cast<uintptr_t>(t.g) % 16) == 0)) {
+        // One pass: each thread loads its STAT_TILE / ST_THREADS elements and sums x,
+        // x^2 and |x| (fp32 over each loaded group, pairwise; fp64 across groups).
+        constexpr int V = vec_elems<GT>();
+        constexpr int NL = STAT_TILE / (V * ST_THREADS);
         constexpr double NT = (double)(V * NL);        // elements per thread
         u32x4 raw[NL];
 #pragma unroll
-        for (int k = 0; k < NL; ++k) raw[k] = load_piece(line, k * ST_THREADS + (int)threadIdx.x);
-        if (16u * threadIdx.x < off)
-            raw[0] = splice(load_piece(line, STAT_TILE / V + (int)threadIdx.x), raw[0], off - 16u * threadIdx.x);
-        // the tile's element in place e of this thread's piece k
-        const auto pos = [&](int k, int e) {
-            const int i = V * (k * ST_THREADS + (int)threadIdx.x) + e - offe;
-            return base + (i < 0 ? i + STAT_TILE : i);
-        };
+        for (int k = 0; k < NL; ++k) raw[k] = load_raw<GT>(t.g, base + V * ((int64_t)k * ST_THREADS + threadIdx.x));
+        // the element in place e of this thread's load k
+        const auto pos = [&](int k, int e) { return base + V * ((int64_t)k * ST_THREADS + threadIdx.x) + e; };
         double sx = 0.0, sq = 0.0, ab = 0.0;
 #pragma unroll
         for (int k = 0; k < NL; ++k) {
@@ -313,52 +381,14 @@ __global__ __launch_bounds__(ST_THREADS) void stats_partial_kernel(const StatDes
         }
         return;
     }
-    // A ragged last tile: per-element fp64 sums, the tile mean, then a second pass (from L2)
-    // for the squared deviations from it.  RC pieces a thread are in flight at a time: all of
-    // them would take 132 registers and halve the whole tiles' occupancy.
-    const uint32_t cnt = (uint32_t)(t.numel - base);   // elements of the tile
-    const int pieces = (int)((off + cnt * ES + 15u) / 16u);
-    const auto each = [&](auto &&f) {
-        constexpr int RC = 4;
-#pragma unroll 1
-        for (int w0 = (int)threadIdx.x; w0 < pieces; w0 += RC * ST_THREADS) {
-            u32x4 raw[RC];
-#pragma unroll
-            for (int k = 0; k < RC; ++k) {
-                const int w = w0 + k * ST_THREADS;
-                raw[k] = u32x4{0u, 0u, 0u, 0u};
-                if (w < pieces && (uint32_t)(w + 1) * 16u > off) raw[k] = *(const ST_GLOBAL u32x4 *)(line + 16 * (int64_t)w);
-            }
-#pragma unroll
-            for (int k = 0; k < RC; ++k) {
-                float x[V];
-                widen<GT>(raw[k], x);
-                const int i0 = V * (w0 + k * ST_THREADS) - offe;
-#pragma unroll
-                for (int e = 0; e < V; ++e) f(x[e], (uint32_t)(i0 + e) < cnt);
-            }
+    const void *g = static_cast<const char *>(t.g) + base * (GT == GT_F32 ? 4 : 2);
+    if constexpr (OFF16) {
+        if (left >= STAT_TILE) {
+            whole_f64<GT>(g, partials + 4 * tile, lds3, lds2);
+            return;
         }
-    };
-    double s[3] = {0.0, 0.0, 0.0};      // sum g, sum g^2, sum |g|
-    each([&](float x, bool in) { acc(s[0], s[1], s[2], in ? x : 0.0f); });
-    block_sum<3>(s, lds3);
-    const double n_t = (double)cnt;
-    const float c = (float)(s[0] / n_t);
-    double dv[2] = {0.0, 0.0};          // sum d, sum d^2 with d = g - c
-    each([&](float x, bool in) {
-        const double dd = in ? (double)x - (double)c : 0.0;
-        dv[0] += dd;
-        dv[1] = fma(dd, dd, dv[1]);
-    });
-    block_sum<2>(dv, lds2);
-    if (threadIdx.x == 0) {
-        // d = g - c is exact in fp64, so M2 = sum d^2 - (sum d)^2 / n and sum g = n c + sum d
-        // are as accurate as the tile's spread allows (non-finite g: the first pass's sum)
-        partials[4 * tile + 0] = fabs(dv[0]) <= __DBL_MAX__ ? fma(n_t, (double)c, dv[0]) : s[0];
-        partials[4 * tile + 1] = dv[1] - dv[0] * (dv[0] / n_t);
-        partials[4 * tile + 2] = s[1];
-        partials[4 * tile + 3] = s[2];
     }
+    ragged_f64<GT>(g, (uint32_t)left, partials + 4 * tile, lds3, lds2);
 }
 
 // fp32 value of a sum of non-negative terms as an fp32 accumulator holds it:
@@ -449,16 +479,18 @@ hipError_t launch_scores(const float *stats, const float *mean, int n, const flo
     return hipGetLastError();
 }
 
-hipError_t launch_grad_stats(const StatDesc *d, const long long *tb, int n, long long tiles, int grad_dt,
+hipError_t launch_grad_stats(const StatDesc *d, const long long *tb, int n, long long tiles, int grad_dt, bool off16,
                              double *partials, float *out, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
     if (tiles > 0) {
-        const dim3 grid((unsigned)tiles), block(ST_THREADS);
+        const auto partial = [&](auto kernel) {
+            kernel<<<dim3((unsigned)tiles), dim3(ST_THREADS), 0, s>>>(d, n, tb, partials);
+        };
         switch (grad_dt) {
-        case GT_F32: stats_partial_kernel<GT_F32><<<grid, block, 0, s>>>(d, n, tb, partials); break;
-        case GT_BF16: stats_partial_kernel<GT_BF16><<<grid, block, 0, s>>>(d, n, tb, partials); break;
-        default: stats_partial_kernel<GT_F16><<<grid, block, 0, s>>>(d, n, tb, partials); break;
+        case GT_F32: partial(off16 ? stats_partial_kernel<GT_F32, true> : stats_partial_kernel<GT_F32, false>); break;
+        case GT_BF16: partial(off16 ? stats_partial_kernel<GT_BF16, true> : stats_partial_kernel<GT_BF16, false>); break;
+        default: partial(off16 ? stats_partial_kernel<GT_F16, true> : stats_partial_kernel<GT_F16, false>); break;
         }
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;

@@ -110,6 +110,64 @@ def test_tiles_at_any_place_in_their_line(dtype, offsets, values):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n", [32768, 65536])
+def test_sums_off_16_bytes_are_fp64_at_every_place(dtype, n):
+    """Whole tiles of tensors that do not start on 16 bytes: mean g^2 is the correctly rounded one (fp64
+    sums of the fp32 squares; fp32 sums of neighbours lose s^2 = 0.992 * 2^-24 beside 1, by where a
+    group of 4 or 8 starts), and all statistics have the same bits wherever in its line the tensor
+    starts; the same bits again at every multiple of 16 bytes."""
+    print(f"case: grad_stats sums off 16 bytes {dtype} n={n}", flush=True)
+    es = 4 if dtype == torch.float32 else 2
+    s = 2.0 ** -12 * 0.99609375
+    x = torch.tensor([1.0, s, s, 0.0] if es == 4 else [1.0, s, s, 0.0, s, 0.0, 0.0, 0.0]).repeat(n)[:n].to(dtype).to(DEV)
+    noise = (torch.randn(n, generator=torch.Generator().manual_seed(n)) * 1e-3).to(dtype).to(DEV)
+    offsets = range(0, 128 // es)
+    buf = torch.zeros(2 * len(offsets) * (n + 64 + 128), dtype=dtype, device=DEV)
+    assert buf.data_ptr() % 128 == 0
+    vs, o = [], 0
+    for t in (x, noise):
+        for off in offsets:
+            buf[o + off:o + off + n] = t
+            vs.append(buf[o + off:o + off + n])
+            o += n + 64 + 128 // es - (n + 64) % (128 // es)
+    got = mdq_hip.grad_stats(vs).cpu().numpy().view(np.uint32).reshape(2, len(offsets), 3)
+    whole = np.array([off * es % 16 == 0 for off in offsets])
+    for k in range(2):
+        assert np.unique(got[k][whole], axis=0).shape[0] == 1, "depends on the multiple of 16 bytes"
+        assert np.unique(got[k][~whole], axis=0).shape[0] == 1, "depends on the place in the line"
+    x64 = x.double()
+    want = np.float32((x64 * x64).sum().item() / n)     # the squares are exact in fp32, n a power of two
+    assert want > np.float32(1.0 / (4 if es == 4 else 8))
+    assert (got[0][~whole][:, 2] == want.view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shift", [1, 2, 3, 6])
+def test_grads_at_any_byte_address(dtype, shift):
+    """The C entry takes grads that do not lie on a multiple of their element size: the bits are those
+    of the same values at an element offset."""
+    print(f"case: grad_stats byte shift {shift} {dtype}", flush=True)
+    es = 4 if dtype == torch.float32 else 2
+    rng = np.random.default_rng(shift)
+    ptrs, numels, keep, vs = [], [], [], []
+    for n in (5, 1000, 32768, 40_000, 65_536):
+        x = torch.from_numpy((rng.standard_t(3, n) * 1e-3).astype(np.float32)).to(dtype)
+        raw = torch.zeros(n * es + 64, dtype=torch.uint8, device=DEV)
+        raw[shift:shift + n * es] = x.view(torch.uint8).to(DEV)
+        buf = torch.zeros(n + 8, dtype=dtype, device=DEV)
+        buf[1:1 + n] = x.to(DEV)
+        keep.append(raw)
+        ptrs.append(raw.data_ptr() + shift)
+        numels.append(n)
+        vs.append(buf[1:1 + n])
+    out = torch.empty(len(ptrs), 3, device=DEV)
+    p, m = np.array(ptrs, dtype=np.uint64), np.array(numels, dtype=np.int64)
+    mdq_hip.check(mdq_hip.lib().stq_multi_tensor_grad_stats(p.ctypes.data, m.ctypes.data, len(ptrs), mdq_hip.dtype_code(dtype),
+                                                            out.data_ptr(), torch.cuda.current_stream(DEV).cuda_stream))
+    assert torch.equal(out.view(torch.int32), mdq_hip.grad_stats(vs).view(torch.int32))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_nonfinite_grads_match_oracle(dtype):
     """NaN, +-inf and (fp32) overflowing squares in some tensors of a launch: the kernel gives the
     oracle's NaN / inf entries (pinned to the reference's torch expression on the CPU), finite
