@@ -211,7 +211,8 @@ int stq_multi_tensor_grad_stats(const void *const *grads, const int64_t *numels,
  *   out[n_tensors + i] = r_l.
  * t[i] = step / tau per tensor, or NULL where all tensors share t_all.  All
  * arrays are device memory; out (2 n_tensors floats) and ema must not overlap
- * the inputs.
+ * the inputs.  With n_tensors == 0 only ema is written (stats and out may be
+ * NULL; nothing at all if mean and ema are NULL too).
  *
  * Replaces the per-tensor score of MDQAdamWSimple
  * (/root/reference/CUDA/stquant_opt_simple.py:433-466).

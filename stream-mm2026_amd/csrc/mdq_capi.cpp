@@ -960,11 +960,11 @@ int stq_decision_scores(const float *stats, const float *mean, int n_tensors, co
                         float one_minus_alpha, float *out, float *ema, void *stream)
 {
     g_err.clear();
-    if (n_tensors < 0 || (n_tensors > 0 && (!stats || !mean || !out || !ema)))
+    if (n_tensors < 0 || !mean != !ema || (n_tensors > 0 && (!stats || !mean || !out)))
         return fail(STQ_ERR_INVALID, "decision_scores: bad statistics or output");
     if ((n_ema == nullptr) != (r_ema == nullptr) || (n_ema == nullptr) != (v_ema == nullptr))
         return fail(STQ_ERR_INVALID, "decision_scores: all three EMAs or none");
-    if (n_tensors == 0) return STQ_OK;
+    if (!ema) return STQ_OK;   // no tensors and no EMAs
     const hipError_t e = mdq::launch_scores(stats, mean, n_tensors, t, t_all, n_ema, r_ema, v_ema, alpha,
                                             one_minus_alpha, out, ema, reinterpret_cast<hipStream_t>(stream));
     return e == hipSuccess ? STQ_OK : hip_fail(e, "decision_scores launch");

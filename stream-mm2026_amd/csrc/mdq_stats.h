@@ -27,7 +27,7 @@ static_assert(sizeof(StatDesc) == 32, "StatDesc layout");
 hipError_t launch_grad_stats(const StatDesc *d, const long long *tile_begin, int n, long long tiles,
                              int grad_dt, bool off16, double *partials, float *out, hipStream_t s);
 
-// The bit decision's scores of n > 0 tensors from their statistics stats[3n] and the mean of
+// The bit decision's scores of n >= 0 tensors from their statistics stats[3n] and the mean of
 // those over the tensors: out[0 .. n) the scores, out[n .. 2n) the r_l; ema[3] the EMAs
 // (n, r, v) after this decision, a * mean + b * previous (the mean where n_ema is null).
 // t: the tensors' step / tau, or null where all share t_all.

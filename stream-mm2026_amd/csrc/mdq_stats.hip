@@ -474,7 +474,8 @@ __global__ __launch_bounds__(256) void scores_kernel(const float *__restrict__ s
 hipError_t launch_scores(const float *stats, const float *mean, int n, const float *t, float t_all, const float *n_ema,
                          const float *r_ema, const float *v_ema, float a, float b, float *out, float *ema, hipStream_t s)
 {
-    scores_kernel<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s>>>(stats, mean, n, t, t_all, n_ema, r_ema, v_ema,
+    // without tensors one workgroup still writes the EMAs
+    scores_kernel<<<dim3((unsigned)(n > 0 ? (n + 255) / 256 : 1)), dim3(256), 0, s>>>(stats, mean, n, t, t_all, n_ema, r_ema, v_ema,
                                                                          a, b, out, ema);
     return hipGetLastError();
 }

@@ -469,6 +469,8 @@ def decision_scores(stats: torch.Tensor, mean: torch.Tensor, t: Sequence[float],
     of the n scores and the n ``r_l``, and the ``[3]`` EMAs (n, r, v) after folding in ``mean``.
     ``t``: each tensor's step / tau; ``ema``: the EMAs so far (three 0-d tensors), or None at the
     first decision.  The same fp32 operations as the reference's (stquant_opt_simple.py:433-466)."""
+    if stats.dim() != 2 or stats.shape[1] != 3:
+        raise RuntimeError(f"decision_scores: statistics must be [n, 3], got {list(stats.shape)}")
     n, dev = stats.shape[0], stats.device
     if dev.type != "cuda" or len(t) != n:
         raise RuntimeError("decision_scores: statistics on a CUDA device and one t per tensor")
@@ -479,13 +481,11 @@ def decision_scores(stats: torch.Tensor, mean: torch.Tensor, t: Sequence[float],
         raise RuntimeError("decision_scores: a mean of 3 and three EMAs")
     out = torch.empty(2 * n, dtype=torch.float32, device=dev)
     new = torch.empty(3, dtype=torch.float32, device=dev)
-    if n == 0:
-        return out, new
-    same = t.count(t[0]) == n
-    ts = None if same else torch.tensor(t, dtype=torch.float32, device=dev)
+    t_all = t[0] if n else 0.0
+    ts = None if t.count(t_all) == n else torch.tensor(t, dtype=torch.float32, device=dev)
     e = [x.data_ptr() for x in ema] if ema is not None else [None] * 3
-    launch(dev, lib().stq_decision_scores, stats.data_ptr(), mean.data_ptr(), n, _ptr(ts), t[0], *e, alpha, 1 - alpha,
-           out.data_ptr(), new.data_ptr())
+    launch(dev, lib().stq_decision_scores, _ptr(stats), mean.data_ptr(), n, _ptr(ts), t_all, *e, alpha, 1 - alpha,
+           _ptr(out), new.data_ptr())
     return out, new
 
 

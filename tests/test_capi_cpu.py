@@ -211,3 +211,24 @@ def test_host_tensors_are_rejected_before_any_launch():
 def test_state_tensors_on_another_device_are_rejected():
     with pytest.raises(RuntimeError, match="scale_m must be on the params' device"):
         mdq_hip.MultiTensorPlan([_state(dev="meta")], 128)
+
+
+@pytest.mark.parametrize("shape", [(4,), (12,), (4, 1), (4, 2), (4, 4), (4, 3, 1), (0,), (0, 2)])
+def test_decision_scores_wants_three_statistics_a_tensor(shape):
+    with pytest.raises(RuntimeError, match=r"must be \[n, 3\]"):
+        mdq_hip.decision_scores(torch.zeros(shape), torch.zeros(3), [1.0] * shape[0], None, 0.9)
+
+
+def scores_call(stats=FAKE, mean=FAKE, n=1, ema=(None, None, None), out=FAKE, new=FAKE):
+    return mdq_hip.lib().stq_decision_scores(stats, mean, n, None, 1.0, *ema, 0.9, 0.1, out, new, None)
+
+
+@pytest.mark.parametrize("kw", [dict(n=-1), dict(stats=None), dict(mean=None), dict(out=None), dict(new=None),
+                                dict(ema=(FAKE, None, FAKE)), dict(n=0, mean=None), dict(n=0, new=None)])
+def test_decision_scores_argument_errors(kw):
+    assert scores_call(**kw) == 1
+    assert err().startswith("decision_scores: ")
+
+
+def test_decision_scores_without_tensors_and_emas_is_a_no_op():
+    assert scores_call(stats=None, mean=None, n=0, out=None, new=None) == 0

@@ -255,6 +255,20 @@ def test_decision_launch_is_the_torch_chain(n, first, same_step):
     np.testing.assert_array_equal(host, torch.cat((want, stats[:, 1])).cpu().numpy())
 
 
+@pytest.mark.parametrize("first", [True, False])
+def test_decision_without_tensors_folds_the_emas(first):
+    """No tensors: no scores, and the EMAs with this mean folded in, as with tensors."""
+    print(f"case: decision_scores n=0 first={first}", flush=True)
+    opt = MDQAdamWSimple([torch.nn.Parameter(torch.zeros(8, device=DEV))], alpha=0.83)
+    mean = torch.tensor([1e-3, 2.0, 3e-7], device=DEV)
+    ema = None
+    if not first:
+        ema = opt.n_ema, opt.r_ema, opt.v_global_ema = torch.tensor([2e-3, 1.5, 1e-6], device=DEV).unbind(0)
+    out, new = mdq_hip.decision_scores(torch.empty(0, 3, device=DEV), mean, [], ema, 0.83)
+    assert out.shape == (0,)
+    assert torch.equal(new, torch.stack(opt._folded_ema(mean)))
+
+
 def test_optimizer_fused_stats_same_decisions():
     print("case: optimizer grad_stats fused vs reference", flush=True)
     shapes = [(700, 13), (4096,), (129,), (3, 1000), (50_000,)]
