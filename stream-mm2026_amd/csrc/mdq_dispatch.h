@@ -10,18 +10,28 @@
 
 namespace mdq {
 
+template <int SRC, int DST, int GT, int LOG2B, bool SR, bool VIEWS>
+static void launch_waves(const MdqDesc *d, int n, long long tiles, unsigned long long *prof, const StepArgs &sa,
+                         hipStream_t s)
+{
+    // the compact tile_begin array follows the n descriptors in the same buffer
+    const long long *tb = reinterpret_cast<const long long *>(d + n);
+    constexpr int big = waves_per_simd<SRC, DST, GT, LOG2B, SR, VIEWS, false>(true);
+    constexpr int small = waves_per_simd<SRC, DST, GT, LOG2B, SR, VIEWS, false>(false);
+    if (big == small || beyond_cache<SRC, DST, GT, LOG2B>(tiles))
+        hipLaunchKernelGGL((mdq_step_kernel<SRC, DST, GT, LOG2B, SR, VIEWS, big>), dim3((unsigned)tiles),
+                           dim3(Cfg<LOG2B>::THREADS), 0, s, d, tb, n, prof, sa);
+    else
+        hipLaunchKernelGGL((mdq_step_kernel<SRC, DST, GT, LOG2B, SR, VIEWS, small>), dim3((unsigned)tiles),
+                           dim3(Cfg<LOG2B>::THREADS), 0, s, d, tb, n, prof, sa);
+}
+
 template <int SRC, int DST, int GT, int LOG2B, bool SR>
 static hipError_t launch_one(const MdqDesc *d, int n, long long tiles, unsigned long long *prof,
                              const StepArgs &sa, bool views, hipStream_t s)
 {
-    // the compact tile_begin array follows the n descriptors in the same buffer
-    const long long *tb = reinterpret_cast<const long long *>(d + n);
-    if (views)
-        hipLaunchKernelGGL((mdq_step_kernel<SRC, DST, GT, LOG2B, SR, true>), dim3((unsigned)tiles),
-                           dim3(Cfg<LOG2B>::THREADS), 0, s, d, tb, n, prof, sa);
-    else
-        hipLaunchKernelGGL((mdq_step_kernel<SRC, DST, GT, LOG2B, SR, false>), dim3((unsigned)tiles),
-                           dim3(Cfg<LOG2B>::THREADS), 0, s, d, tb, n, prof, sa);
+    if (views) launch_waves<SRC, DST, GT, LOG2B, SR, true>(d, n, tiles, prof, sa, s);
+    else launch_waves<SRC, DST, GT, LOG2B, SR, false>(d, n, tiles, prof, sa, s);
     return hipGetLastError();
 }
 
@@ -66,8 +76,14 @@ template <int ST, int GT, int LOG2B, bool SR>
 static hipError_t launch_arg(const MdqDesc &d, long long tiles, unsigned long long *prof, const StepArgs &sa,
                              hipStream_t s)
 {
-    hipLaunchKernelGGL((mdq_step_kernel_one<ST, GT, LOG2B, SR>), dim3((unsigned)tiles), dim3(Cfg<LOG2B>::THREADS),
-                       0, s, d, prof, sa);
+    constexpr int big = waves_per_simd<ST, ST, GT, LOG2B, SR, true, true>(true);
+    constexpr int small = waves_per_simd<ST, ST, GT, LOG2B, SR, true, true>(false);
+    if (big == small || beyond_cache<ST, ST, GT, LOG2B>(tiles))
+        hipLaunchKernelGGL((mdq_step_kernel_one<ST, GT, LOG2B, SR, big>), dim3((unsigned)tiles),
+                           dim3(Cfg<LOG2B>::THREADS), 0, s, d, prof, sa);
+    else
+        hipLaunchKernelGGL((mdq_step_kernel_one<ST, GT, LOG2B, SR, small>), dim3((unsigned)tiles),
+                           dim3(Cfg<LOG2B>::THREADS), 0, s, d, prof, sa);
     return hipGetLastError();
 }
 

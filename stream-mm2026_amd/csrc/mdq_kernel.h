@@ -1411,43 +1411,77 @@ __device__ __forceinline__ void mdq_step_tile_any(const MdqDesc &d, long long ti
 // 4-bit codes with stochastic rounding keep 7 (6: LLaMA-7B +0.8 %, views B = 64 +1.2 %); most
 // other stochastic kernels need 73-85 VGPRs and hold 5-6 anyway.
 //
-// Steps on wider codes and at B = 1024 are capped by the bytes their waves ask for at once: a
-// wave issues all loads of its tile together, so W waves per SIMD keep W x 256 lanes x the lane's
-// load bytes (p, grads, codes) in flight per CU, and beyond about 104 KB more of them cost
-// bandwidth.  Measured on GPT-2 small, W = the compiler's own count -> the rule's:
-//   32-bit codes, fp32 grads (128 B a lane)   6 -> 3  601.2 -> 561.2 us at B = 128, 594.4 -> 564.1 at 256
-//   32-bit codes, bf16 grads (112 B)          6 -> 3  545.8 -> 524.4, 534.7 -> 517.2
-//   16-bit codes, fp32 grads (96 B)           5-7 -> 4  409.2 -> 396.1, 398.0 -> 390.8
-//   16-bit codes, bf16 grads (80 B)           5-7 -> 5  364.0 -> 360.6, 358.0 -> 358.0
-// At B = 1024 (twice the elements per lane) three waves are needed for their own arithmetic, and
-// more are too many: 4-bit 284.8 -> 275.8 (fp32 grads), 237.2 -> 232.4 (bf16), 8-bit 330.6 -> 316.4,
-// 279.8 -> 277.7, 16-bit 418.3 -> 403.8; two waves are slower (305.5, 281.1, 328.7, 325.7, 417.3)
-// except for 32-bit codes (224-256 B a lane): 622.1 -> 567.1, bf16 631.8 -> 551.8.
-// 8-bit codes with fp32 grads (80 B) as packed views, nearest rounding: 6 -> 5 waves 950.7 -> 929.8 us
-// (257 ragged tensors, B = 64), level otherwise.  As views 16-bit codes gain most (1418 -> 1320 us).
-// The one-tensor kernel (ONE) mostly runs on tensors that stay in cache, where 16-bit steps need the
-// waves for their arithmetic (4,194,304 params: 16.0 us, 16.2 by the rule): they keep the compiler's
-// count there, and 8-bit steps six waves.
-// Storage-changing steps follow the same rule with the wider side's codes, between 3 and 5 waves
-// (6 and 7 before): one LLaMA-7B layer, B = 128, nearest: 16 -> 4 fp32 grads 568 -> 548 us, 8 -> 16 589 ->
-// 580, 32 -> 16 832 -> 775, bf16 grads 32 -> 4 640 -> 621, 8 -> 4 420 -> 415; 16 -> 4 and back with
-// bf16 grads, B = 256: level to -1 % (run to run).
+// Steps on wider codes ask for more bytes per wave.  A wave issues all loads of its tile together, so
+// W waves per SIMD keep W x 256 lanes x the lane's load bytes (p, grads, codes) in flight per CU; from
+// about 104 KB on, more of them cost bandwidth (`fit` below).  Times relative to the compiler's own
+// count, from forced counts 2 to 7 in one process, in turn; GPT-2 small (beyond the cache) / 100 ragged
+// tensors (in it), B = 64 and 256, nearest:
+//   32-bit codes, fp32 grads (128 B a lane)  3 waves  0.89, 0.90 / 0.95, 0.98   2: 0.89, 0.90 / 0.99, 1.02
+//   32-bit codes, bf16 grads (112 B)         3        0.96, 0.95 / 0.97, 0.99   2: 1.01, 1.01 / 1.03, 1.06
+//   16-bit codes, fp32 grads (96 B)          4        0.95, 0.97 / 0.97, 0.99   3: 0.94, 1.01 / 0.98, 1.03
+//   16-bit codes, bf16 grads (80 B)          5        0.98, 0.99 / 0.98, 1.00   4: 0.97, 1.00 / 0.96, 0.99
+// 16-bit codes with fp32 grads as views take 5 from B = 128 on: 0.99-1.00 in and beyond the cache,
+// where 4 take 1.01-1.05 (at B = 64 0.94 beyond it).
+// What this does not hold for was measured too, each cell with its own count:
+// - B = 1024 (twice the elements a lane): its arithmetic needs the waves while the data is in the
+//   last-level cache.  4-bit, fp32 grads: 3 waves 1.15 at 59 MB a launch, 1.00 at 117 MB, 0.98 from 235 MB
+//   on; 16-bit 1.19 at 84 MB, 1.02 at 168 MB, 1.00 at 294 MB, 0.97 at 1 GB; one 32-bit tensor, bf16, 2
+//   waves 1.06 at 109 MB (0.94 with the compiler's 3), 0.95 (0.96) at 327 MB, 0.93 (1.01) at 1.3 GB.  So
+//   the cap there applies to launches beyond the cache (`big`) and to lanes of 144 bytes and more; bf16
+//   4- and 8-bit steps lose 8 % with 3 waves on GPT-2 small.
+// - 8-bit codes with fp32 grads as packed views, nearest: 5 waves for big launches.  Heavy-tailed grads
+//   (257 ragged tensors) gain 1 to 2.4 %, normal ones lose 1 to 2.8 %; in the cache 5 cost 3.4 %.
+// - One-tensor 16-bit steps in the cache keep the compiler's count (5 waves: +1 to +2 % at B = 128, 512).
+// - B = 8 to 32 spend their time on the scales, which the waves' own lanes fetch, and run best with
+//   fewer: 8-bit table launches 4 waves (B = 16 0.93 / 0.97, B = 32 0.94 / 0.98), 16-bit 4 (0.92 / 0.94),
+//   4-bit 5 at B = 16 (0.96 / 1.00); views and one-tensor steps keep their counts, but for stochastic
+//   one-tensor steps at B = 16 and 32: 5 (6: +1 to +4 %).
+// - Storage-changing steps, one LLaMA-7B layer and the two sets above: to or from 32 bits 3 waves (fp32
+//   grads 32 -> 4 0.89, to 16 0.90, to 32 0.94-0.98), 4 where they narrow to 8 or 4 bits with 16-bit grads
+//   (32 -> 4 0.95-0.97 / 1.00, with 3 1.04 / 1.08) or fp32 32 -> 4 in the cache (0.98; 3: 1.02); to 16 bits
+//   4 with fp32 grads (0.92-0.98), 5 with 16-bit ones (0.96-0.99); 16 -> 8 the same, but 6 with 16-bit
+//   grads from B = 128 on and 16 -> 4 one more (16-bit grads, B = 256: 6 waves 1.00, 5 1.02, 4 1.10); 4 <-> 8
+//   bits 6 as before (5: 1.01 to 1.04), 5 for fp32 4 -> 8 from B = 128 on (0.97-0.99).
 template <int SRC, int DST, int GT, int LOG2B, bool SR, bool VIEWS, bool ONE>
-constexpr int waves_per_simd()
+constexpr int waves_per_simd(bool big)
 {
+    constexpr bool f32 = GT == GT_F32;
     constexpr auto code_bytes = [](int st) { return code_size(st) * (st == ST_P4 ? 1 : 2); };
-    constexpr int codes = code_bytes(SRC) > code_bytes(DST) ? code_bytes(SRC) : code_bytes(DST);
-    constexpr int w = 104 * 1024 / (256 * Cfg<LOG2B>::EPL * (4 + (GT == GT_F32 ? 4 : 2) + codes));
-    if (SRC != DST) return w < 3 ? 3 : w > 5 ? 5 : w;
-    if ((SRC == ST_S16 && !ONE) || SRC == ST_S32 || LOG2B == 10) {
-        constexpr int least = SRC == ST_S32 && LOG2B == 10 ? 2 : 3;
-        return w < least ? least : w > 7 ? 7 : w;
+    if (SRC != DST) {
+        constexpr int widest = code_bytes(SRC) > code_bytes(DST) ? code_bytes(SRC) : code_bytes(DST);
+        if (widest == 8) return DST >= ST_S16 || (f32 && (big || DST == ST_S8)) ? 3 : 4;
+        if (widest == 4) return DST == ST_P4 ? (f32 ? 5 : 6) : f32 ? 4 : DST == ST_S16 || LOG2B == 6 ? 5 : 6;
+        return f32 && DST == ST_S8 && LOG2B >= 7 ? 5 : SR ? 7 : 6;
     }
-    if (SRC == ST_S8) return VIEWS && !ONE && !SR && GT == GT_F32 ? 5 : 6;
+    constexpr int lane = Cfg<LOG2B>::EPL * (4 + (f32 ? 4 : 2) + code_bytes(SRC));   // bytes a lane loads
+    constexpr int fit = 104 * 1024 / (256 * lane) < 7 ? 104 * 1024 / (256 * lane) : 7;
+    constexpr bool table_views = VIEWS && !ONE;
+    constexpr bool tiny = LOG2B >= 3 && LOG2B <= 5;          // B = 8, 16, 32
+    if (LOG2B == 10) {
+        if (big && lane >= 224) return 2;
+        if (big && lane >= (table_views ? 192 : 144) && f32) return 3;
+    } else if (SRC == ST_S32) {
+        return fit;
+    } else if (SRC == ST_S16) {
+        if (ONE && !big) return SR && LOG2B >= 4 && LOG2B <= 5 ? 5 : 7;
+        return tiny && !ONE ? 4 : table_views && LOG2B >= 7 && fit < 5 ? 5 : fit;
+    } else if (tiny) {
+        if (ONE && SR && LOG2B >= 4) return 5;
+        if (!VIEWS) return SRC == ST_S8 ? 4 : LOG2B == 4 ? 5 : SR ? 7 : 6;
+    }
+    if (SRC == ST_S8) return big && table_views && !SR && f32 && LOG2B >= 3 && LOG2B < 10 ? fit : 6;
     return !SR && SRC == ST_P4 ? 6 : 7;
 }
 
-// Reserves registers up to the count that leaves room for waves_per_simd waves.
+// Whether a launch over this many tiles moves more than the 256 MB that the last-level cache holds.
+template <int SRC, int DST, int GT, int LOG2B>
+bool beyond_cache(long long tiles)
+{
+    constexpr int codes = code_size(SRC) * (SRC == ST_P4 ? 1 : 2) + code_size(DST) * (DST == ST_P4 ? 1 : 2);
+    return tiles * Cfg<LOG2B>::TILE * (8 + (GT == GT_F32 ? 4 : 2) + codes) > 256ll << 20;
+}
+
+// Reserves registers up to the count that leaves room for W waves per SIMD.
 template <int W>
 __device__ __forceinline__ void occupancy_cap()
 {
@@ -1463,14 +1497,14 @@ __device__ __forceinline__ void occupancy_cap()
 // The launch over a descriptor table: the tile's tensor is the largest t with
 // tile_begin[t] <= tile (tile_begin: compact int64 copy of the descriptors' tile starts, so
 // the ~log2(n_desc) dependent scalar loads hit a few cache lines).
-template <int SRC, int DST, int GT, int LOG2B, bool SR, bool VIEWS>
+template <int SRC, int DST, int GT, int LOG2B, bool SR, bool VIEWS, int W>
 __global__ __launch_bounds__(Cfg<LOG2B>::THREADS) void mdq_step_kernel(const MdqDesc *__restrict__ descs,
                                                                       const long long *__restrict__ tile_begin,
                                                                       int n_desc,
                                                                       unsigned long long *__restrict__ prof,
                                                                       const StepArgs sa)
 {
-    occupancy_cap<waves_per_simd<SRC, DST, GT, LOG2B, SR, VIEWS, false>()>();
+    occupancy_cap<W>();
     using L = StepLds<SRC, DST, GT, LOG2B, SR, VIEWS>;
     __shared__ float lut_s[L::LUT];
     __shared__ int32_t xw_s[6];
@@ -1491,12 +1525,12 @@ __global__ __launch_bounds__(Cfg<LOG2B>::THREADS) void mdq_step_kernel(const Mdq
 // call), and a call on a stream that is capturing a HIP graph records a plain kernel node.
 // The variant with every tile mode (a one-tensor LLaMA-size step runs level with the
 // table-driven kernel).
-template <int SRC, int GT, int LOG2B, bool SR>
+template <int SRC, int GT, int LOG2B, bool SR, int W>
 __global__ __launch_bounds__(Cfg<LOG2B>::THREADS) void mdq_step_kernel_one(const MdqDesc d,
                                                                           unsigned long long *__restrict__ prof,
                                                                           const StepArgs sa)
 {
-    occupancy_cap<waves_per_simd<SRC, SRC, GT, LOG2B, SR, true, true>()>();
+    occupancy_cap<W>();
     using L = StepLds<SRC, SRC, GT, LOG2B, SR, true>;
     __shared__ float lut_s[L::LUT];
     __shared__ int32_t xw_s[6];
