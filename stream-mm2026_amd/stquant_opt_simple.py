@@ -423,8 +423,9 @@ class MDQAdamWSimple(Optimizer):
         hyper-parameters are refreshed.  Plans keep no reference to gradients.
         """
         buckets = OrderedDict()
-        launch_keys = {id(g): (min(int(g["block_size"]), 1024), mdq_hip.rounding_code(g.get("rounding", "nearest")),
-                               int(g.get("seed", 0) or 0)) for _p, g in items}
+        groups = {id(g): g for _p, g in items}
+        launch_keys = {k: (min(int(g["block_size"]), 1024), mdq_hip.rounding_code(g.get("rounding", "nearest")),
+                           int(g.get("seed", 0) or 0)) for k, g in groups.items()}
         for i, (p, group) in enumerate(items):
             state = self.state[p]
             grad = p.grad

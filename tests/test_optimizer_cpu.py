@@ -386,3 +386,19 @@ def test_checkpoint_keeps_codes_bit_identical(bits):
     opt2.step()
     for p, q in zip(params, params2):
         assert torch.equal(p.detach(), q.detach())
+
+
+def test_launch_options_are_formed_once_per_group(monkeypatch):
+    """A step that plans its launches forms a group's block size, rounding and seed once, however many
+    tensors the group has."""
+    params = make_params([(9, 7)] * 8)
+    opt = SimpleCPU([dict(params=params[:5], bits=4), dict(params=params[5:], bits=8)], lr=1e-3, block_size=64)
+    set_grads(params, 0)
+    opt.step()
+    calls = []
+    code = mdq_hip.rounding_code
+    monkeypatch.setattr(mdq_hip, "rounding_code", lambda r: calls.append(r) or code(r))
+    opt._steady = None
+    set_grads(params, 1)
+    opt.step()
+    assert len(calls) == 2
