@@ -401,4 +401,4 @@ def test_launch_options_are_formed_once_per_group(monkeypatch):
     opt._steady = None
     set_grads(params, 1)
     opt.step()
-    assert len(calls) == 2
+    assert calls.count("nearest") == 2, calls      # (a plan takes the code already formed)
