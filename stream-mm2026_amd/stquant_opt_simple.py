@@ -155,6 +155,7 @@ class MDQAdamWSimple(Optimizer):
         self._settled = 0                   # rows of the last decision taken from torch's reductions
         self._profile = _PhaseProfile()
 
+    _made = None    # (statistics, ``_decision`` on them) between settling and the decision of a step
     # launch-plan class of ``_run_kernels`` (a test harness substitutes its own executor)
     _plan_cls = mdq_hip.MultiTensorPlan
     # False: layout changes of CUDA tensors run as torch ops per tensor instead of device launches
@@ -195,17 +196,12 @@ class MDQAdamWSimple(Optimizer):
         """``[n, 3]`` stats of all grads: one fused launch per grad dtype (``'fused'``, settled on
         the reference's torch reductions near the thresholds, and ``'exact'``), or the reference's
         per-tensor torch reductions (``'reference'``, stquant_opt_simple.py:427-431)."""
-        return self._stats_and_decision(grads, steps, tau)[0]
-
-    def _stats_and_decision(self, grads, steps=None, tau=None):
-        """``_all_grad_stats``, and the decision (``_decision``) that settling them already made on
-        exactly these statistics (None where it made none, or on others)."""
         if self.grad_stats != "reference" and grads and grads[0].is_cuda:
             stats = mdq_hip.grad_stats(grads)
             if self.grad_stats == "fused" and steps is not None:
-                return self._settle(stats, grads, steps, tau)
-            return stats, None
-        return torch.stack([self._compute_grad_stats(g.float()) for g in grads]), None
+                stats = self._settle(stats, grads, steps, tau)
+            return stats
+        return torch.stack([self._compute_grad_stats(g.float()) for g in grads])
 
     def _decision(self, stats, mean, steps, tau):
         """``(scores, host, ema)`` of these statistics and their mean, which the EMAs fold in: the
@@ -227,8 +223,8 @@ class MDQAdamWSimple(Optimizer):
         """The fused statistics, with the rows of the tensors whose width the fused and the
         reference statistics could decide differently replaced by the reference's torch
         reductions: scores within SETTLE_MARGIN of a threshold (provisional scores against the
-        EMAs this decision would fold in), near-constant tensors, and non-finite rows.  With them
-        the provisional decision, where no row was replaced."""
+        EMAs this decision would fold in), near-constant tensors, and non-finite rows.  Where no
+        row is replaced, the provisional decision is left in ``_made``, with its statistics."""
         prov = self._decision(stats, stats.mean(dim=0), steps, tau)
         sc, r = prov[1][:len(grads)], prov[1][len(grads):]
         near = np.zeros(len(grads), dtype=bool)
@@ -236,12 +232,13 @@ class MDQAdamWSimple(Optimizer):
             near |= np.abs(sc - lo) < self.SETTLE_MARGIN
         redo = np.nonzero(near | (r < self.NEAR_CONSTANT_R) | ~np.isfinite(sc) | ~np.isfinite(r))[0].tolist()
         if not redo:
-            return stats, prov
+            self._made = stats, prov
+            return stats
         stats = stats.clone()
         stats[torch.as_tensor(redo, device=stats.device)] = torch.stack(
             [self._compute_grad_stats(grads[i].float()) for i in redo])
         self._settled = len(redo)
-        return stats, None
+        return stats
 
     def _scores(self, stats_tensor, steps, tau, ema=None):
         """The reference's per-tensor score (stquant_opt_simple.py:446-466) for all tensors at
@@ -284,8 +281,11 @@ class MDQAdamWSimple(Optimizer):
         steps = [st["step"] for st in states]
         tau = self.param_groups[0]["tau"]
         self._settled = 0
+        self._made = None
         with _Stopwatch(dev) as sw:
-            stats, made = self._stats_and_decision([p.grad for p, _g in work], steps, tau)
+            stats = self._all_grad_stats([p.grad for p, _g in work], steps, tau)
+        made, self._made = self._made, None
+        made = made[1] if made is not None and made[0] is stats else None
         lt["mdq_grad_stats_ms"] = sw.ms
         lt["mdq_grad_stats_settled"] = self._settled
         across = dist.is_available() and dist.is_initialized()

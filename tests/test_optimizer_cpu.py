@@ -402,3 +402,20 @@ def test_launch_options_are_formed_once_per_group(monkeypatch):
     set_grads(params, 1)
     opt.step()
     assert calls.count("nearest") == 2, calls      # (a plan takes the code already formed)
+
+
+def test_the_decision_takes_the_statistics_of_the_method():
+    """``_all_grad_stats`` is what a deciding step scores, also where a subclass replaces it."""
+    class Louder(SimpleCPU):
+        def _all_grad_stats(self, grads, steps=None, tau=None):
+            stats = super()._all_grad_stats(grads, steps, tau).clone()
+            stats[0] *= 2.0 ** 10
+            stats[1:] *= 2.0 ** -10
+            return stats
+
+    params = make_params([(40, 40)] * 4)
+    set_grads(params, 3)
+    opt = Louder(params, lr=1e-3)
+    opt.step()
+    widths = [opt.state[p]["current_bit"] for p in params]
+    assert widths[0] > max(widths[1:]), widths
