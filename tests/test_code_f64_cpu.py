@@ -1,7 +1,8 @@
 """``mdq_code_f64`` (csrc/mdq_math.h, the requant of 17..32-bit codes) compiled for the CPU against the
-reference's own arithmetic, an IEEE double division and round half away (stquant_kernel.cu:366-381):
-exact ties and their neighbours, quotients next to 1/2 and to powers of two, quotients beyond the
-range, zeros, subnormals, infinities and NaN."""
+reference's own arithmetic, an IEEE double division and round half away, clamped, NaN as 0
+(stquant_kernel.cu:366-381): exact ties and their neighbours, quotients next to 1/2 and to powers of
+two, quotients beyond the range, zeros, subnormals, infinite and NaN divisors.  The two kinds of pairs
+that it is not for, and that no block of a step has, are labelled as such."""
 import ctypes
 import os
 import subprocess
@@ -42,9 +43,8 @@ def reference(u, d, lim):
     with np.errstate(all="ignore"):
         q = u.astype(np.float64) / d.astype(np.float64)
         t = np.trunc(q)
-        k = t + (np.abs(q - t) >= 0.5)
-    k = np.where(np.isfinite(u) & np.isfinite(d), k, 0.0)
-    return np.clip(k, 0.0, lim).astype(np.uint32)
+        k = np.where(np.isinf(q), q, t + (np.abs(q - t) >= 0.5))
+    return np.clip(np.where(np.isnan(q), 0.0, k), 0.0, lim).astype(np.uint32)
 
 
 @pytest.mark.parametrize("bits", [17, 24, 31, 32])
@@ -71,7 +71,15 @@ def test_equals_the_fp64_division_and_round(codes, bits):
 def test_edges(codes):
     f = np.float32
     fmax, tiny, inf, nan = np.finfo(f).max, f(1e-45), f(np.inf), f(np.nan)
-    u = np.array([0, 0, tiny, tiny, fmax, fmax, fmax, inf, 1, inf, nan, 1, nan, 3, fmax], f)
-    d = np.array([1e-12, inf, 1e-12, fmax, 1e-12, fmax, 2 * tiny, inf, inf, 1, 1, nan, nan, 2, 1], f)
+    u = np.array([0, 0, tiny, tiny, fmax, fmax, fmax, inf, inf, 1, nan, 1, nan, 3, fmax], f)
+    d = np.array([1e-12, inf, 1e-12, fmax, 1e-12, fmax, 2 * tiny, inf, nan, inf, 1, nan, nan, 2, 1], f)
     for lim in (2.0 ** 32 - 1, 2.0 ** 31, 2.0 ** 17 - 1):
         np.testing.assert_array_equal(codes(u, d, lim), reference(u, d, lim))
+
+
+def test_pairs_that_no_block_has(codes):
+    """An infinite u over a finite d, and u > 0 over d = 0: 0, where the division would clamp to lim.  The
+    divisor of a block is infinite or NaN where an element is, and at least 1e-12 over the range."""
+    u, d = np.array([np.inf, 1.0], np.float32), np.array([1.0, 0.0], np.float32)
+    assert codes(u, d, 2.0 ** 31).tolist() == [0, 0]
+    assert reference(u, d, 2.0 ** 31).tolist() == [2 ** 31, 2 ** 31]
