@@ -156,7 +156,8 @@ MDQ_HD float mdq_round_half_away(float u, float d, float inv_lo, float hd)
 // a whole lim in [0, 2^32), u infinite only where d is infinite or NaN; 0 where the quotient is
 // NaN, as the reference's (int) of NaN on its target gives (stquant_kernel.cu:366,376).  In the step
 // d is the block's scale, its largest u over the width's range, plus 1e-12: above 0, and infinite
-// or NaN where an element is infinite.  (Infinite u over a finite d, and u > 0 over 0, give 0 here and lim by division.)
+// or NaN where an element is infinite.  (Infinite u over a finite d, and u > 0 over 0, give 0 here
+// and lim by division.)
 // y = RN(1 / d): q0 = RN(u y) is within 2^-51 of u / d, its residual r = u - q0 d is exact (a
 // multiple of the two operands' last places, below 2^26 of them), and q0 + r y lies within
 // 2^-104 of u / d.  The quotient of two 24-bit significands keeps 2^-78 away from every midpoint

@@ -182,7 +182,7 @@ __device__ __forceinline__ void tile_f64(uint32_t cnt, Each each, double *__rest
 }
 
 // A whole tile at any byte address.  Each thread keeps its elements from the first pass for the
-// second (a 16-bit pair in one register), 113 registers in fp32 and 92 in 16 bits; read again
+// second (a 16-bit pair in one register), 113 registers in fp32 and 85-88 in 16 bits; read again
 // instead, 8 in flight as for a ragged tile, the 257 ragged tensors take 350 us in place of 234 in
 // fp32 and 227 in place of 184 in bf16.  16 loads at a time: 32 and 64 take 196 and 203 us in bf16.
 template <int GT>
@@ -222,12 +222,13 @@ __device__ __forceinline__ void whole_f64(const void *g, double *__restrict__ pa
 }
 
 // A ragged last tile of cnt elements at any byte address, read once a pass (the second time from
-// L2) with 8 loads a thread in flight: 16 take the kernel from 6 waves per SIMD to 5.
+// L2) with 16 loads a thread in flight: 24 spill at 6 waves per SIMD, 8 run 100 ragged tensors in
+// 24.5 us in place of 23.9.
 template <int GT>
 __device__ __forceinline__ void ragged_f64(const void *g, uint32_t cnt, double *__restrict__ partial, double (*lds3)[3],
                                            double (*lds2)[2])
 {
-    constexpr int G = 8;
+    constexpr int G = 16;
     tile_f64(cnt, [&](auto &&f) {
 #pragma unroll 1
         for (uint32_t i0 = threadIdx.x; i0 < cnt; i0 += G * ST_THREADS) {
@@ -245,11 +246,12 @@ __device__ __forceinline__ void ragged_f64(const void *g, uint32_t cnt, double *
 
 // OFF16: some tensor of the launch starts off 16 bytes and has a whole tile.  An instance of its
 // own: whole_f64's registers would leave the 16-byte path 4 waves per SIMD (257 aligned ragged
-// bf16 tensors 119 -> 135 us).
+// bf16 tensors 119 -> 135 us).  The counts are asked for: left to itself the compiler gives the
+// other instance 84 registers and 5 waves, and this one's loads less room (199 us in place of 191).
 template <int GT, bool OFF16>
-__global__ __launch_bounds__(ST_THREADS) void stats_partial_kernel(const StatDesc *__restrict__ d, int n,
-                                                                   const long long *__restrict__ tb,
-                                                                   double *__restrict__ partials)
+__global__ __launch_bounds__(ST_THREADS) __attribute__((amdgpu_waves_per_eu(OFF16 ? 4 : 6)))
+void stats_partial_kernel(const StatDesc *__restrict__ d, int n, const long long *__restrict__ tb,
+                          double *__restrict__ partials)
 {
     __shared__ double lds4[ST_WAVES][4];
     __shared__ double lds3[ST_WAVES][3];
