@@ -265,7 +265,8 @@ class MultiTensorPlan:
         gdt, eadt, easqdt = self.codes
         L = lib()
         fn = L.stq_multi_tensor_mdq_adamw_noalloc if noalloc else L.stq_multi_tensor_mdq_adamw
-        launch(self.device, fn, self.arr.__array_interface__["data"][0], self.n, gdt, eadt, easqdt,
+        # (the address by .ctypes: __array_interface__ describes the 23 fields each time, 5 us)
+        launch(self.device, fn, self.arr.ctypes.data, self.n, gdt, eadt, easqdt,
                self.block_size, self.rounding, self.seed, prof_ptr, prof_n)
 
 

@@ -9,6 +9,8 @@ steady steps in both rounding modes, tensors with different step counts (no kern
 constants), two tensor sets alternating, a grad buffer that moves, another stream, and ring
 slots taken in between by other entry points.
 """
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -159,3 +161,21 @@ def test_random_sequence_of_launches():
             mdq_hip.grad_stats([x])
     print(f"uploads over 36 launches: {ups}", flush=True)
     assert 3 <= ups < 36
+
+
+def test_a_steady_launch_enters_few_python_functions():
+    """``MultiTensorPlan.run`` of a plan as it stands: no description of the descriptor list's fields
+    (24 functions a call) on the way to the launch."""
+    print("case: python functions of a plan's launch", flush=True)
+    s = Set(41)
+    entries = [c.entry(t, 1, 4, tensor_id=i) for i, (c, t) in enumerate(zip(s.cases, s.tg))]
+    plan = mdq_hip.MultiTensorPlan(entries, B)
+    plan.run()
+    calls = []
+    sys.setprofile(lambda frame, event, arg: calls.append(frame.f_code.co_name) if event == "call" else None)
+    try:
+        plan.run()
+    finally:
+        sys.setprofile(None)
+    torch.cuda.synchronize()
+    assert len(calls) <= 16, calls
