@@ -47,8 +47,8 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 # Unbound forms for map() over a launch's tensor lists: a list of n tensors costs n calls from C
 # and no bytecode per tensor.  The calls whose host time exceeds their kernels': convert_codes over
-# GPT-2 small's 148 tensors 305 -> 156 us, fused_step on one small tensor 11.6 -> 7.8 us, a plan of
-# 600 small tensors (with its constants formed once, mdq_capi.cpp) 43.5 -> 23.4 us.
+# GPT-2 small's 148 tensors 305 -> 156 us, fused_step on one small tensor 11.6 -> 7.8 us (with the
+# checks in one look and launch() in place of a device guard).
 _address = torch.Tensor.data_ptr
 _numel = torch.Tensor.numel
 _contiguous = torch.Tensor.is_contiguous
@@ -272,32 +272,42 @@ class MultiTensorPlan:
 
 def _pack_entries(entries: Sequence[TensorState]):
     n = len(entries)
-    arr = np.zeros(n, dtype=STQ_TENSOR_DTYPE)
     if n == 0:
-        return arr, (0, 0, 0)
+        return np.zeros(0, dtype=STQ_TENSOR_DTYPE), (0, 0, 0)
     e0 = entries[0]
     dev = e0.p.device
     gdt, eadt, easqdt = e0.grad.dtype, e0.exp_avg.dtype, e0.exp_avg_sq.dtype
-    cols = {k: [getattr(e, k) for e in entries] for k in _ENTRY_TENSORS}
-    # column by column: the row-wise checks run only to name what is wrong
-    every = [t for c in cols.values() for t in c]
-    if not ({*map(_device_of, every)} == {dev.index} and all(map(_contiguous, every))
-            and all({*map(_dtype, cols[k])} == {dt} for k, dt in (("p", torch.float32), ("grad", gdt),
-                                                                   ("exp_avg", eadt), ("exp_avg_sq", easqdt)))):
+    if n < 4:
+        # row by row: the columns below cost 10 us before the first tensor (host time of 1 / 2 / 4 /
+        # 148 tensors row by row 8 / 14 / 25 / 1018 us, by columns 13 / 18 / 27 / 591)
         _check_entries(entries, dev, gdt, eadt, easqdt)
-    for k, c in cols.items():
-        arr[k] = [*map(_address, c)]
-        arr["numel" if k == "p" else k + "_numel"] = [*map(_numel, c)]
+        rows = [(e.p.data_ptr(), e.grad.data_ptr(), e.exp_avg.data_ptr(),
+                 e.exp_avg_sq.data_ptr() if e.exp_avg_sq.numel() else 0,
+                 e.scale_m.data_ptr(), e.scale_v.data_ptr(), e.v_min.data_ptr(),
+                 e.p.numel(), e.grad.numel(), e.exp_avg.numel(), e.exp_avg_sq.numel(),
+                 e.scale_m.numel(), e.scale_v.numel(), e.v_min.numel(),
+                 float(e.beta1), float(e.beta2), float(e.lr), float(e.weight_decay), float(e.eps), int(e.step), int(e.bits),
+                 int(e.tensor_id) & 0xFFFFFFFF, int(e.elem_offset)) for e in entries]
+        return np.array(rows, dtype=STQ_TENSOR_DTYPE), (dtype_code(gdt), dtype_code(eadt), dtype_code(easqdt))
+    cols = [*zip(*map(_entry_tensors, entries))]
+    # column by column: the row-wise checks run only to name what is wrong
+    every = [t for c in cols for t in c]
+    if not ({*map(_device_of, every)} == {dev.index} and all(map(_contiguous, every))
+            and [{*map(_dtype, c)} for c in cols[:4]] == [{torch.float32}, {gdt}, {eadt}, {easqdt}]):
+        _check_entries(entries, dev, gdt, eadt, easqdt)
+    ptrs, numels = [*map(_address, every)], [*map(_numel, every)]
+    beta1, beta2, lr, weight_decay, eps, step, bits, ids, offset = zip(*map(_entry_numbers, entries))
+    rows = zip(*(ptrs[k:k + n] for k in range(0, 7 * n, n)), *(numels[k:k + n] for k in range(0, 7 * n, n)),
+               *(map(float, x) for x in (beta1, beta2, lr, weight_decay, eps)), map(int, step), map(int, bits),
+               [int(i) & 0xFFFFFFFF for i in ids], map(int, offset))
+    arr = np.array([*rows], dtype=STQ_TENSOR_DTYPE)
     arr["exp_avg_sq"][arr["exp_avg_sq_numel"] == 0] = 0
-    for k in ("beta1", "beta2", "lr", "weight_decay", "eps"):
-        arr[k] = [float(getattr(e, k)) for e in entries]
-    for k in ("step", "bits", "elem_offset"):
-        arr[k] = [int(getattr(e, k)) for e in entries]
-    arr["tensor_id"] = [int(e.tensor_id) & 0xFFFFFFFF for e in entries]
     return arr, (dtype_code(gdt), dtype_code(eadt), dtype_code(easqdt))
 
 
 _ENTRY_TENSORS = ("p", "grad", "exp_avg", "exp_avg_sq", "scale_m", "scale_v", "v_min")
+_entry_tensors = attrgetter(*_ENTRY_TENSORS)
+_entry_numbers = attrgetter("beta1", "beta2", "lr", "weight_decay", "eps", "step", "bits", "tensor_id", "elem_offset")
 
 
 def _check_entries(entries, dev, gdt, eadt, easqdt) -> None:

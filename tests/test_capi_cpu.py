@@ -4,7 +4,9 @@ and rejects bad arguments with the reference's messages before touching a GPU
 import ctypes
 import os
 import re
+import sys
 
+import numpy as np
 import pytest
 import torch
 
@@ -232,3 +234,47 @@ def test_decision_scores_argument_errors(kw):
 
 def test_decision_scores_without_tensors_and_emas_is_a_no_op():
     assert scores_call(stats=None, mean=None, n=0, out=None, new=None) == 0
+
+
+def python_calls(fn):
+    """Python functions entered while fn() runs (comprehensions and generators count)."""
+    calls = []
+    sys.setprofile(lambda frame, event, arg: calls.append(frame.f_code.co_name) if event == "call" else None)
+    try:
+        fn()
+    finally:
+        sys.setprofile(None)
+    return calls
+
+
+def tensor_state(n=500, B=128):
+    nb = -(-n // B)
+    return mdq_hip.TensorState(torch.zeros(n), torch.zeros(n), torch.zeros(n, dtype=torch.int8), torch.zeros(n, dtype=torch.uint8),
+                               torch.zeros(nb), torch.zeros(nb), torch.zeros(nb), 5, 8, 1e-4, 0.9, 0.999, 1e-8, 0.01, 7)
+
+
+def test_packing_one_tensor_enters_few_python_functions():
+    """One tensor is packed row by row: a list, its check, three dtype codes."""
+    entries = [tensor_state()]
+    calls = python_calls(lambda: mdq_hip._pack_entries(entries))
+    assert len(calls) <= 8, calls
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 9])
+def test_packed_rows_hold_the_entries(n):
+    """Few tensors (row by row) and more (by columns): every field, packed nibbles' absent v codes among them."""
+    entries = [tensor_state(500 + k) for k in range(n)]
+    for k, e in enumerate(entries):
+        e.step, e.bits, e.lr, e.tensor_id, e.elem_offset = 3 + k, 8 - k % 3, 1e-3 * (k + 1), -1 - k, 128 * k
+        if n % 2:
+            e.exp_avg, e.exp_avg_sq = e.exp_avg_sq, torch.empty(0, dtype=torch.uint8)
+    arr, dtypes = mdq_hip._pack_entries(entries)
+    assert dtypes == tuple(map(mdq_hip.dtype_code, (torch.float32, entries[0].exp_avg.dtype, torch.uint8)))
+    for e, r in zip(entries, arr):
+        for k in ("p", "grad", "exp_avg", "exp_avg_sq", "scale_m", "scale_v", "v_min"):
+            t = getattr(e, k)
+            assert r[k] == (t.data_ptr() if t.numel() else 0)
+            assert r["numel" if k == "p" else k + "_numel"] == t.numel()
+        for k in ("beta1", "beta2", "lr", "weight_decay", "eps"):
+            assert r[k] == np.float32(getattr(e, k))
+        assert (r["step"], r["bits"], r["tensor_id"], r["elem_offset"]) == (e.step, e.bits, e.tensor_id & 0xFFFFFFFF, e.elem_offset)
