@@ -1428,10 +1428,12 @@ __device__ __forceinline__ void mdq_step_tile_any(const MdqDesc &d, long long ti
 //   on; 16-bit 1.19 at 84 MB, 1.02 at 168 MB, 1.00 at 294 MB, 0.97 at 1 GB; one 32-bit tensor, bf16, 2
 //   waves 1.06 at 109 MB (0.94 with the compiler's 3), 0.95 (0.96) at 327 MB, 0.93 (1.01) at 1.3 GB.  So
 //   the cap there applies to launches beyond the cache (`big`) and to lanes of 144 bytes and more; bf16
-//   4- and 8-bit steps lose 8 % with 3 waves on GPT-2 small.
+//   4- and 8-bit steps lose 8 % with 3 waves on GPT-2 small, and 8-bit table launches with fp32 grads
+//   gain nothing (1.00 to 1.02; one tensor of 100 M params 1.01, with 4 waves 1.04).
 // - 8-bit codes with fp32 grads as packed views, nearest: 5 waves for big launches.  Heavy-tailed grads
 //   (257 ragged tensors) gain 1 to 2.4 %, normal ones lose 1 to 2.8 %; in the cache 5 cost 3.4 %.
-// - One-tensor 16-bit steps in the cache keep the compiler's count (5 waves: +1 to +2 % at B = 128, 512).
+// - One-tensor 16-bit steps in the cache keep the compiler's count (5 waves: +1 to +2 % at B = 128, 512),
+//   but for stochastic ones up to B = 256, which take 5 (more: +2 to +6 % at B = 128).
 // - B = 8 to 32 spend their time on the scales, which the waves' own lanes fetch, and run best with
 //   fewer: 8-bit table launches 4 waves (B = 16 0.93 / 0.97, B = 32 0.94 / 0.98), 16-bit 4 (0.92 / 0.94),
 //   4-bit 5 at B = 16 (0.96 / 1.00); views and one-tensor steps keep their counts, but for stochastic
@@ -1459,11 +1461,11 @@ constexpr int waves_per_simd(bool big)
     constexpr bool tiny = LOG2B >= 3 && LOG2B <= 5;          // B = 8, 16, 32
     if (LOG2B == 10) {
         if (big && lane >= 224) return 2;
-        if (big && lane >= (table_views ? 192 : 144) && f32) return 3;
+        if (big && lane >= (table_views ? 192 : 144) && f32 && (ONE || SRC != ST_S8)) return 3;
     } else if (SRC == ST_S32) {
         return fit;
     } else if (SRC == ST_S16) {
-        if (ONE && !big) return SR && LOG2B >= 4 && LOG2B <= 5 ? 5 : 7;
+        if (ONE && !big) return SR && LOG2B >= 4 && LOG2B <= 8 ? 5 : 7;
         return tiny && !ONE ? 4 : table_views && LOG2B >= 7 && fit < 5 ? 5 : fit;
     } else if (tiny) {
         if (ONE && SR && LOG2B >= 4) return 5;
